@@ -578,7 +578,7 @@ __device__ __forceinline__ void run_att(const Params& p, Smem<S>& sm, const int*
             kv_load<S>(rkv, p, 0, g, nxt.t0 / 32, (nxt.t1 - nxt.t0 + 31) / 32, wave_id());
             gain_load_qk<S>(rkv, p, 0);
           }
-        }, lw))
+        }, lw, !cur.on && o0 < 0))  // a split that a later token of the launch opens: no role in this token
       return;
     if constexpr ((MODE & 2) != 0) trace_end(p, t);
   }

@@ -15,6 +15,8 @@ import pytest
 import torch
 
 from megakernel_amd import _lib
+from megakernel_amd.bridge import MegakernelEngine
+from megakernel_amd.weights import DeviceWeights
 from megakernel_amd.config import BASELINE, QWEN3_06B, TINY
 from oracle import qwen3_ref, synth
 
@@ -524,6 +526,33 @@ def test_bridge_benchmark_and_sweep():
         for r in res:
             assert r["tok_per_sec"] > 0 and r["latency_us"] > 0 and 0 < r["bw_util"] < 1.0
         assert eng.pos == 500 + 8
+    finally:
+        eng.close()
+        dw.free()
+
+
+def test_resident_launch_opens_an_attention_split():
+    """A resident launch whose later tokens need one more attention split than
+    its first ones: the workgroups of that split have no role before it opens,
+    and must not score the LM head from an x word of an earlier layer (4-bit
+    tags repeat every 15 phases = 3 layers).  The resident tokens equal the
+    per-token path's, whose launches hold exactly their token's splits."""
+    shape = BASELINE.with_(n_layers=7, vocab=8192)
+    dw = DeviceWeights(shape, 77, gain_std=0.1)
+    eng = MegakernelEngine(shape=shape, max_seq=512, device_weights=dw)
+    try:
+        eng.set_attention_chunk(64)
+        for i, start in enumerate([58, 122, 186, 250, 314, 378] * 2):
+            eng.fill_kv_synthetic(start, 5 + i)
+            n = 10
+            assert eng.decode_kernel_for(n) == _lib.KERNEL_CLASS
+            got = eng.decode_many(11 + 97 * i, n)
+            eng.set_pos(start)
+            tok, want = 11 + 97 * i, []
+            for _ in range(n):
+                tok = eng.decode_token(tok)
+                want.append(tok)
+            assert got == want, f"start {start}: resident {got}, per token {want}"
     finally:
         eng.close()
         dw.free()
