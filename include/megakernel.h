@@ -133,7 +133,8 @@ float megakernel_last_kernel_ms(void* handle);
 /* Number of resident workgroups of the decode kernel (one per CU). */
 int megakernel_grid_size(void* handle);
 
-/* Minimum positions per attention work item (default 512). */
+/* Minimum positions per attention work item (default 512; 256 for head_dim
+ * 128). */
 int megakernel_set_attention_chunk(void* handle, int chunk_min);
 
 /* Above this many attention splits per kv head (default 20: contexts beyond

@@ -478,13 +478,13 @@ __device__ __forceinline__ void kv_load_paced(KV<S, K8>& r, const Params& p, int
     kv_load<S>(r, p, layer, g, b0, nb, wave_id());
     return;
   }
-  // one block of the wave's KVB per step (its K and V^T loads together)
+  // one block of the wave's per step (its K and V^T loads together)
   constexpr int D = S::D;
   const unsigned l = lane_id();
   const long long base = kt_base(p, layer, g, S::NKV, D);
   const int bi = wave_id();
 #pragma unroll
-  for (int q = 0; q < KVB; ++q) {
+  for (int q = 0; q < KV<S, K8>::NB; ++q) {
     const int bq = bi + q * NW;
     const int blk = b0 + (bq < nb ? bq : 0);
     if constexpr (K8) {

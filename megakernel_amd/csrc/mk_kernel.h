@@ -42,6 +42,13 @@ constexpr int NW = NT / kWave;
 // Two per wave halves the attention splits (and so the partials every O
 // workgroup merges) against one, at the cost of a longer block step.
 constexpr int KVB = MK_KV_BLOCKS;
+// Blocks of a shape: two of head_dim 64 are 64 registers per lane; two of
+// head_dim 128 would be 128, which the kernels do not have beside that shape's
+// weight blocks (the spread kernel spilled 732 registers per lane), so it
+// takes one (with batches of four splits in the O phase's merge: 1,080 -> 460
+// us per token at 700 positions).
+template <class S>
+constexpr int kv_blocks() { return S::D <= 64 ? KVB : 1; }
 // Cache policy of the LM-head stream (buffer-load aux bits): plain loads on
 // 80 % of it and non-temporal loads on the rest measured fastest (part of the
 // plain-loaded share is served from the memory-side cache across tokens).
@@ -822,13 +829,14 @@ __device__ __forceinline__ int first_item(int wg, int off, int G) { return (wg +
 // [t0, t1); wave w takes the item's blocks w, w + NW, ...
 template <class S, bool K8 = false>
 struct KV {
+  static constexpr int NB = kv_blocks<S>();  // blocks
   static constexpr int KC = S::D / 32;  // k-steps of the score product
   static constexpr int DT = S::D / 16;  // dim tiles of the output product
   // 8 values per lane and operand: bf16 (u32x4) or, for an FP8 cache, e4m3 codes (u32x2)
   using Reg = typename std::conditional<K8, u32x2, u32x4>::type;
-  Reg k[KVB][2][KC];  // K of the wave's blocks: [block][16-position half][k-step]
-  Reg v[KVB][DT];     // V^T of the blocks: [block][dim tile]
-  float sk[K8 ? KVB : 1][2], sv[K8 ? KVB : 1][2];  // FP8: scales of the lane's score positions
+  Reg k[NB][2][KC];   // K of the wave's blocks: [block][16-position half][k-step]
+  Reg v[NB][DT];      // V^T of the blocks: [block][dim tile]
+  float sk[K8 ? NB : 1][2], sv[K8 ? NB : 1][2];  // FP8: scales of the lane's score positions
   uint16_t gn[S::D / kWave];  // QK-norm gain(s) of this lane's dim(s) for its wave's head
 };
 
@@ -858,7 +866,7 @@ __device__ __forceinline__ u32x4 buf_ld_kv(__amdgpu_buffer_rsrc_t rs, unsigned v
   return __builtin_amdgcn_raw_buffer_load_b128(rs, voff, 0u, 16 | 2);
 }
 
-// Loads this wave's KVB blocks of an item starting at block index `bi`
+// Loads this wave's NB blocks of an item starting at block index `bi`
 // (item blocks bi, bi + NW, ...; blocks past the item's nb repeat a valid
 // block and are masked by the caller).
 template <class S, bool K8>
@@ -867,7 +875,7 @@ __device__ __forceinline__ void kv_load(KV<S, K8>& r, const Params& p, int layer
   const unsigned l = lane_id();
   const long long base = kt_base(p, layer, g, S::NKV, D);
 #pragma unroll
-  for (int q = 0; q < KVB; ++q) {
+  for (int q = 0; q < KV<S, K8>::NB; ++q) {
     const int bq = bi + q * NW;
     const int blk = b0 + (bq < nb ? bq : 0);
     if constexpr (K8) {  // byte index = element index of the bf16 layout
@@ -906,7 +914,7 @@ __device__ __forceinline__ void kv_load(KV<S, K8>& r, const Params& p, int layer
 template <class S, bool K8>
 __device__ __forceinline__ void kv_forget(KV<S, K8>& r) {
 #pragma unroll
-  for (int q = 0; q < KVB; ++q) {
+  for (int q = 0; q < KV<S, K8>::NB; ++q) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -916,7 +924,7 @@ __device__ __forceinline__ void kv_forget(KV<S, K8>& r) {
   }
   if constexpr (K8) {
 #pragma unroll
-    for (int q = 0; q < KVB; ++q)
+    for (int q = 0; q < KV<S, K8>::NB; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         r.sk[q][h] = __builtin_nondeterministic_value(r.sk[q][h]);
@@ -1120,7 +1128,7 @@ template <class S, int MODE>
 __device__ bool attention_compute(const Params& p, Smem<S>& sm, KV<S, (MODE & 8) != 0>& kvr, int layer, int pos,
                                   int g, int s, int nsplit, int t0, int t1, unsigned tg, int tt) {
   constexpr bool K8 = (MODE & 8) != 0;
-  constexpr int D = S::D, GQA = S::GQA, KC = KV<S, K8>::KC, DT = KV<S, K8>::DT;
+  constexpr int D = S::D, GQA = S::GQA, KC = KV<S, K8>::KC, DT = KV<S, K8>::DT, NB = KV<S, K8>::NB;
   static_assert(GQA <= 4, "q heads of a group fit the 16 MFMA rows (4 per head)");
   if (!attention_prologue<S, MODE>(p, sm, kvr, layer, pos, g, t0 <= pos && pos < t1, tg, tt)) return false;
   evt(p, tt, layer, EV_ATT_ROPE);
@@ -1136,13 +1144,13 @@ __device__ bool attention_compute(const Params& p, Smem<S>& sm, KV<S, (MODE & 8)
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int b0 = t0 / 32, nb = (t1 - t0 + 31) / 32;
-  // groups of KVB blocks (w + NW * (KVB * gi + q)); the first group was
+  // groups of NB blocks (w + NW * (NB * gi + q)); the first group was
   // prefetched, later ones (long contexts) are loaded here
-  for (int bi = w; bi < nb; bi += KVB * NW) {
+  for (int bi = w; bi < nb; bi += NB * NW) {
     if (bi != w) kv_load<S>(kvr, p, layer, g, b0, nb, bi);
     // the block holding pos takes K / V of pos from LDS
 #pragma unroll
-    for (int q = 0; q < KVB; ++q) {
+    for (int q = 0; q < NB; ++q) {
       const int bp = 32 * (b0 + bi + q * NW);
       if (bi + q * NW < nb && bp <= pos && pos < bp + 32) {
         const int rp = pos - bp;
@@ -1177,14 +1185,14 @@ __device__ bool attention_compute(const Params& p, Smem<S>& sm, KV<S, (MODE & 8)
       }
     }
     // scores: lane (rg, c16) gets head rg at positions 32 (b0 + bi + q NW) + 16 h + c16
-    float sc[KVB][2];
+    float sc[NB][2];
     float bmax = -INFINITY;
 #pragma unroll
-    for (int q = 0; q < KVB; ++q)
+    for (int q = 0; q < NB; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         f32x4 d4 = f32x4{0.f, 0.f, 0.f, 0.f};
-        // a block past the item (the wave has fewer blocks than KVB) is all
+        // a block past the item (the wave has fewer blocks than NB) is all
         // -inf below: its products are skipped (a wave-uniform branch)
         if (bi + q * NW < nb) {
 #pragma unroll
@@ -1207,7 +1215,7 @@ __device__ bool attention_compute(const Params& p, Smem<S>& sm, KV<S, (MODE & 8)
     m = mn;
     float bsum = 0.f;
 #pragma unroll
-    for (int q = 0; q < KVB; ++q)
+    for (int q = 0; q < NB; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         sc[q][h] = __expf(sc[q][h] - mn);
@@ -1218,7 +1226,7 @@ __device__ bool attention_compute(const Params& p, Smem<S>& sm, KV<S, (MODE & 8)
     // LDS operations of one wave complete in order; the other rows stay 0)
     if (rg < GQA) {
 #pragma unroll
-      for (int q = 0; q < KVB; ++q)
+      for (int q = 0; q < NB; ++q)
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
           // FP8 cache: the V row's scale enters with the weight (the sum above stays unscaled)
@@ -1230,15 +1238,15 @@ __device__ bool attention_compute(const Params& p, Smem<S>& sm, KV<S, (MODE & 8)
         }
     }
     asm volatile("" ::: "memory");
-    u32x4 pa[KVB];
+    u32x4 pa[NB];
 #pragma unroll
-    for (int q = 0; q < KVB; ++q) pa[q] = *reinterpret_cast<const u32x4*>(&sm.pb[w][c16][32 * q + 8 * rg]);
+    for (int q = 0; q < NB; ++q) pa[q] = *reinterpret_cast<const u32x4*>(&sm.pb[w][c16][32 * q + 8 * rg]);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[dt][i] *= alpha;
 #pragma unroll
-      for (int q = 0; q < KVB; ++q) {
+      for (int q = 0; q < NB; ++q) {
         if (bi + q * NW < nb) {  // a skipped block has weight 0: no product
           u32x4 vb;
           if constexpr (K8) vb = fp8x8_to_bf16x8_scaled(kvr.v[q][dt], 1.0f);  // V scales ride on the weights
@@ -1471,7 +1479,10 @@ __device__ __forceinline__ int fetch_attn_any(const Params& p, const u64* part, 
   if (nsplit <= 2) return fetch_attn_core<S, 2>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev);
   if (nsplit == 3) return fetch_attn_core<S, 3>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev);
   if (nsplit <= 8) return fetch_attn_core<S, 4>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev);
-  return fetch_attn_core<S, 8>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev);
+  if constexpr (S::QD / 2 > NT)  // two pairs per thread: a batch of 8 would hold 64 words
+    return fetch_attn_core<S, 4>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev);
+  else
+    return fetch_attn_core<S, 8>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev);
 }
 
 // Workgroup-synchronous form (spread kernel): a barrier before (every wave is
