@@ -148,8 +148,8 @@ int megakernel_set_attention_merge(void* handle, int merge_min);
  * kernel has one shape).  MK_KERNEL_AUTO (default): the class-specialised
  * kernel -- every workgroup keeps one role class for the launch and loads a
  * role's next weights right after computing it -- whenever a role table
- * holds all attention items of the launch (up to 4 splits per kv head on the
- * BASELINE and TINY presets), else the spread kernel; MK_KERNEL_SPREAD: always
+ * holds all attention items of the launch (up to 8 splits per kv head, 4 on
+ * the QWEN3_06B preset), else the spread kernel; MK_KERNEL_SPREAD: always
  * the spread kernel.  megakernel_decode_kernel_for reports which kernel a
  * launch of n_tokens from the current position would use. */
 #define MK_KERNEL_AUTO 0

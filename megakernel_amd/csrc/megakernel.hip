@@ -295,6 +295,7 @@ struct ShapeInfo {
   long long u_layer, off_qkv, off_o, off_gu, off_down;
   int srows_layer, srow_qkv, srow_o, srow_gu, srow_down;  // FP8 row-scale offsets per layer
   int norm_stride, norm_attn, norm_q, norm_k, norm_ffn;
+  int q_wg;        // QKV blocks per workgroup of the class kernel
   int part_words;  // words of one attention item's published partial
 };
 
@@ -303,7 +304,7 @@ static ShapeInfo shape_info() {
   return ShapeInfo{S::H, S::NQ, S::NKV, S::D, S::F, S::QD, S::KVD, S::QKV, S::GQA,
                    S::U_LAYER, S::OFF_QKV, S::OFF_O, S::OFF_GU, S::OFF_DOWN,
                    S::SROWS_LAYER, S::SROW_QKV, S::SROW_O, S::SROW_GU, S::SROW_DOWN,
-                   S::NORM_STRIDE, S::NORM_ATTN, S::NORM_Q, S::NORM_K, S::NORM_FFN, part_words<S>()};
+                   S::NORM_STRIDE, S::NORM_ATTN, S::NORM_Q, S::NORM_K, S::NORM_FFN, S::Q_WG, part_words<S>()};
 }
 
 // Attention splits per kv head up to which the class kernel has role tables
@@ -315,6 +316,10 @@ constexpr int kMaxClsSplit = 8;
 // class kernel 2,451 tok/s, nine of 512 in the spread kernel 2,261; at 8,192
 // eight of 1,088 lose, 1,957 vs 2,104).
 constexpr int kClsChunkMax = 640;
+// ... of head_dim 128 (four splits; us per token, class / spread kernel: at
+// 1,100 positions, three splits of 384, 417 / 462; at 1,500, four, 436 / 462;
+// at 2,040, four of 512, 560 / 485)
+constexpr int kClsChunkMax128 = 384;
 
 // Role table of the class kernel (mk_cls.h) for `nsplit` attention splits
 // per kv head on G workgroups: attention items (att_o: each with an O block)
@@ -352,17 +357,14 @@ static bool build_roles_as(const ShapeInfo& s, int G, int nsplit, bool att_o, st
       if (!used[next_any]) return used[next_any] = 1, (int)next_any;
     return -1;
   };
-  const int nqg = RBQ < RBF ? RBQ : RBF;
+  const int nq = (RBQ + s.q_wg - 1) / s.q_wg, nqg = nq < RBF ? nq : RBF;
   if (w + nqg > G) return false;
-  for (int i = 0; i < nqg; ++i, ++w) {
-    at(w, RF_CLS) = CLS_QG;
-    at(w, RF_Q) = take_q(w);
-    at(w, RF_G) = i;
-  }
-  for (int i = nqg; i < RBQ; ++i, ++w) {  // QKV blocks without a gate/up partner
+  for (int i = 0; i < nq; ++i, ++w) {  // QKV blocks, with a gate/up pair while they last
     if (w >= G) return false;
-    at(w, RF_CLS) = CLS_Q;
+    at(w, RF_CLS) = i < nqg ? CLS_QG : CLS_Q;
     at(w, RF_Q) = take_q(w);
+    if (s.q_wg == 2) at(w, RF_Q1) = take_q(w);
+    if (i < nqg) at(w, RF_G) = i;
   }
   int d = 0;
   for (int gi = nqg; gi < RBF; ++gi, ++w) {  // gate/up pairs: with a down block while they last
@@ -399,7 +401,19 @@ static bool build_roles_as(const ShapeInfo& s, int G, int nsplit, bool att_o, st
 // Attention-only workgroups when the O blocks fit on the other workgroups
 // (3,133 -> 3,146 tok/s at ctx 1024, alternating runs), else attention
 // workgroups that also take an O block.
+// Shapes with two QKV blocks per workgroup take the first form only, and only
+// with the classes their kernel holds (with the others compiled in it spills;
+// with an O block on the attention workgroups, five to eight splits, it was
+// slower than the spread kernel: 490 against 462 us per token at 1,500).
 static bool build_roles(const ShapeInfo& s, int G, int nsplit, std::vector<int>& rows) {
+  if (s.q_wg == 2) {
+    if (!build_roles_as(s, G, nsplit, false, rows)) return false;
+    for (int w = 0; w < G; ++w) {
+      const int c = rows[(size_t)w * ROLE_INTS + RF_CLS];
+      if (c != CLS_A && c != CLS_QG && c != CLS_DG && c != CLS_O && c != CLS_IDLE) return false;
+    }
+    return true;
+  }
   return build_roles_as(s, G, nsplit, false, rows) || build_roles_as(s, G, nsplit, true, rows);
 }
 
@@ -453,8 +467,11 @@ struct Handle {
   // ([kMaxClsSplit][G][ROLE_INTS] ints); roles_ok[k]: a table for k splits exists
   int* roles = nullptr;
   bool roles_ok[kMaxClsSplit + 1] = {};
+  int cls_split = 0;      // the largest count up to which every table exists
+  int cls_chunk_max = 0;  // the largest chunk a launch takes to stay within it (launch_chunk)
   int kernel_variant = MK_KERNEL_AUTO;
   bool has_cls = false;  // the preset has class-kernel instantiations
+  bool has_w8 = false;   //   with FP8 layer weights too
   int pace_pct = 100;  // class kernel prefetch pacing (environment MK_PACE_PCT at init; 0 = bursts)
 };
 
@@ -545,6 +562,7 @@ static int init_device_state(Handle* h, const char* base, const long long* off, 
     std::vector<int> all((size_t)kMaxClsSplit * h->G * ROLE_INTS, 0), one;
     for (int k = 1; k <= kMaxClsSplit; ++k) {
       h->roles_ok[k] = build_roles(s, h->G, k, one);
+      if (h->roles_ok[k] && h->cls_split == k - 1) h->cls_split = k;
       if (h->roles_ok[k]) std::copy(one.begin(), one.end(), all.begin() + (size_t)(k - 1) * h->G * ROLE_INTS);
     }
     HIPCHK(hipMalloc(&h->roles, all.size() * sizeof(int)), -1);
@@ -608,7 +626,8 @@ static Handle* create(int preset, int vocab, int max_seq) {
     case PRESET_BASELINE:
       h->sh = shape_info<ShapeBaseline>();
       h->launch = launch_decode_baseline;
-      h->has_cls = true;
+      h->has_cls = h->has_w8 = true;
+      h->cls_chunk_max = kClsChunkMax;
       break;
     case PRESET_QWEN3_06B:
       h->sh = shape_info<ShapeQwen3>();
@@ -616,11 +635,14 @@ static Handle* create(int preset, int vocab, int max_seq) {
       // of 256 446 / 460 / 503 / 571, of 512 494 / 505 / 563 / 620)
       h->chunk_min = 256 * kv_blocks<ShapeQwen3>();
       h->launch = launch_decode_qwen3;
+      h->has_cls = true;
+      h->cls_chunk_max = kClsChunkMax128;
       break;
     case PRESET_TINY:
       h->sh = shape_info<ShapeTiny>();
       h->launch = launch_decode_tiny;
-      h->has_cls = true;
+      h->has_cls = h->has_w8 = true;
+      h->cls_chunk_max = kClsChunkMax;
       break;
     default:
       set_err("unknown preset %d", preset);
@@ -679,17 +701,17 @@ static int clear_pair_words(Handle* h) {
 
 // The attention chunk of a launch whose last token sits at position end - 1:
 // the handle's, or, when that needs more splits per kv head than the class
-// kernel's role tables hold while a chunk of at most kClsChunkMax positions
-// would not, the smallest multiple of 32 positions that gives kMaxClsSplit
+// kernel's role tables hold while a chunk of at most cls_chunk_max positions
+// would not, the smallest multiple of 32 positions that gives cls_split
 // splits (a few longer splits in the class kernel beat more splits in the
 // spread kernel).
 static int launch_chunk(const Handle* h, int end) {
   const int c = h->chunk_min;
-  if (!h->has_cls || h->kernel_variant != MK_KERNEL_AUTO || !h->roles_ok[kMaxClsSplit] ||
-      split_count(end, c, h->nsplit_max) <= kMaxClsSplit)
+  if (!h->has_cls || h->kernel_variant != MK_KERNEL_AUTO || h->cls_split == 0 ||
+      split_count(end, c, h->nsplit_max) <= h->cls_split)
     return c;
-  const int c8 = ((end + kMaxClsSplit - 1) / kMaxClsSplit + 31) / 32 * 32;
-  return c8 > c && c8 <= kClsChunkMax ? c8 : c;
+  const int cw = ((end + h->cls_split - 1) / h->cls_split + 31) / 32 * 32;
+  return cw > c && cw <= h->cls_chunk_max ? cw : c;
 }
 
 // One resident launch decoding n tokens starting at h->pos.
@@ -1288,7 +1310,7 @@ int megakernel_set_layer_fp8(void* handle, int enable) {
     mk::set_err("null handle");
     return -1;
   }
-  if (enable && (!h->has_cls || !h->roles_ok[1])) {
+  if (enable && (!h->has_w8 || !h->roles_ok[1])) {
     mk::set_err("FP8 layer weights need the class kernel, which this preset / device does not have");
     return -1;
   }

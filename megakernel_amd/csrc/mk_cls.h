@@ -14,7 +14,8 @@
 //     A    attention (P2)            next K/V after attention (the default
 //                                    where the O blocks fit elsewhere)
 //     ATT  attention (P2) + O (P3)   next K/V and next O after O
-//     QG   QKV (P1) + gate/up (P4)   gate/up after QKV, next QKV after gate/up
+//     QG   QKV (P1, one or two blocks)
+//          + gate/up (P4)            gate/up after QKV, next QKV after gate/up
 //     DG   gate/up (P4) + down (P5)  next gate/up and next down after down
 //     DO   O (P3) + down (P5)        next O and next down after down
 //     O    one or two O blocks (P3)  next O after O
@@ -43,7 +44,7 @@ using GIn = NormInW<S>;
 enum RoleClass : int { CLS_IDLE = 0, CLS_ATT, CLS_QG, CLS_DG, CLS_DO, CLS_O, CLS_Q, CLS_G, CLS_D, CLS_A, CLS_N };
 // Role row: class, then item indices (-1: none).  att: kv head att % NKV,
 // split att / NKV.
-enum RoleField : int { RF_CLS = 0, RF_Q, RF_G, RF_O0, RF_O1, RF_D, RF_ATT, RF_PAD, ROLE_INTS };
+enum RoleField : int { RF_CLS = 0, RF_Q, RF_G, RF_O0, RF_O1, RF_D, RF_ATT, RF_Q1, ROLE_INTS };
 
 // Attention item (kv head g, split s) for n cached positions.
 __device__ __forceinline__ Item att_item_gs(int g, int s, int n, int chunk_min, int nsplit_max) {
@@ -309,18 +310,31 @@ __device__ __forceinline__ bool cls_lm_head(const Params& p, Smem<S>& sm, int t,
 
 // ----------------------------------------------------------- phase bodies
 // P1: QKV block q of layer `layer` from the prefetched rq (inputs: x of the
-// previous layer, or the embedding row at layer 0).
+// previous layer, or the embedding row at layer 0), and block q1 >= 0 from rq1
+// for shapes with two blocks per workgroup (S::Q_WG).
 template <class S, int MODE, class BH>
-__device__ __forceinline__ bool cls_qkv(const Params& p, Smem<S>& sm, const BH& rq, const GIn<S>& gq,
-                                        int t, int layer, int q, int tok, unsigned tg) {
+__device__ __forceinline__ bool cls_qkv(const Params& p, Smem<S>& sm, const BH& rq, const BH& rq1, const GIn<S>& gq,
+                                        int t, int layer, int q, int q1, int tok, unsigned tg) {
   if (layer > 0) {
     fetch_norm_nb<S>(p, p.x, tg - 1u, gq, sm.vec_q, sm.ssw[0], ev_at(t, layer, PS_QKV));
   } else {
     embed_norm_nb<S>(p, tok, gq, sm.vec_q, sm.ssw[0]);
   }
   if constexpr ((MODE & 2) != 0) trace_mark(p, t, PHASES_PER_LAYER * layer + 0, 0);
-  blk_mma(rq, sm.vec_q, sm.red[RED_Q]);
-  const bool ok = store_block<true>(sm.red[RED_Q], p.qkv + q * 16, row_scale(rq), tg, sm.ssw[0], 1.0f / S::H);
+  bool ok;
+  if constexpr (S::Q_WG == 2) {  // the second block's shares: the workgroup has no O block
+    if (q1 >= 0) blk_mma2(rq, rq1, sm.vec_q, sm.red[RED_Q], sm.red[RED_O0]);
+    else blk_mma(rq, sm.vec_q, sm.red[RED_Q]);
+    __syncthreads();
+    ok = !block_aborted();
+    const int w_ = wave_id();
+    if (w_ == PUB_WAVE) qkv_rows<true>(sm.red[RED_Q], p.qkv + q * 16, row_scale(rq), tg, sm.ssw[0], 1.0f / S::H, ok);
+    else if (w_ == PUB_WAVE - 1 && q1 >= 0)
+      qkv_rows<true>(sm.red[RED_O0], p.qkv + q1 * 16, row_scale(rq1), tg, sm.ssw[0], 1.0f / S::H, ok);
+  } else {
+    blk_mma(rq, sm.vec_q, sm.red[RED_Q]);
+    ok = store_block<true>(sm.red[RED_Q], p.qkv + q * 16, row_scale(rq), tg, sm.ssw[0], 1.0f / S::H);
+  }
   if constexpr ((MODE & 2) != 0) trace_mark(p, t, PHASES_PER_LAYER * layer + 0, 1, PUB_WAVE);
   return ok;
 }
@@ -444,10 +458,14 @@ __device__ __forceinline__ void blk_load_at(Blk8<KC>& b, const Params& p, long l
 
 // Weight block loads of one layer.
 template <class S, class BH>
-__device__ __forceinline__ void ld_qkv(BH& rq, GIn<S>& gq, const Params& p, int layer, int q, int units = 0) {
+__device__ __forceinline__ void ld_qkv(BH& rq, BH& rq1, GIn<S>& gq, const Params& p, int layer, int q, int q1,
+                                       int units = 0) {
   gains_load_w(gq, p.norms + (long long)layer * S::NORM_STRIDE + S::NORM_ATTN);
-  blk_load_at(rq, p, (long long)layer * S::U_LAYER + S::OFF_QKV + (long long)q * S::KT_H * 64,
-              (long long)layer * S::SROWS_LAYER + S::SROW_QKV + q * 16, units);
+  const long long u = (long long)layer * S::U_LAYER + S::OFF_QKV, sr = (long long)layer * S::SROWS_LAYER + S::SROW_QKV;
+  blk_load_at(rq, p, u + (long long)q * S::KT_H * 64, sr + q * 16, units);
+  if constexpr (S::Q_WG == 2) {
+    if (q1 >= 0) blk_load_at(rq1, p, u + (long long)q1 * S::KT_H * 64, sr + q1 * 16, units);
+  }
 }
 template <class S, class BH>
 __device__ __forceinline__ void ld_gu(BH& rg, BH& ru, GIn<S>& gf, const Params& p, int layer, int g,
@@ -588,10 +606,10 @@ __device__ __forceinline__ void run_att(const Params& p, Smem<S>& sm, const int*
 template <class S, int MODE, bool HAS_Q, bool HAS_G>
 __device__ __forceinline__ void run_qg(const Params& p, Smem<S>& sm, const int* role) {
   constexpr bool W8 = (MODE & 16) != 0;  // FP8 layer weights
-  const int q = role[RF_Q], gi = role[RF_G];
-  BlkW<S::KC_H, W8> rq, rg, ru;
+  const int q = role[RF_Q], q1 = S::Q_WG == 2 ? role[RF_Q1] : -1, gi = role[RF_G];
+  BlkW<S::KC_H, W8> rq, rq1, rg, ru;
   GIn<S> gq, gf;
-  if constexpr (HAS_Q) ld_qkv<S>(rq, gq, p, 0, q);
+  if constexpr (HAS_Q) ld_qkv<S>(rq, rq1, gq, p, 0, q, q1);
   if constexpr (!HAS_Q && HAS_G) ld_gu<S>(rg, ru, gf, p, 0, gi);
   int tok = p.first_token;
   const unsigned per_token = (unsigned)(PHASES_PER_LAYER * p.n_layers + 1);
@@ -602,14 +620,14 @@ __device__ __forceinline__ void run_qg(const Params& p, Smem<S>& sm, const int* 
     for (int layer = 0; layer < p.n_layers; ++layer) {
       const unsigned tg = tb + (unsigned)(PHASES_PER_LAYER * layer);
       if constexpr (HAS_Q) {
-        if (!cls_qkv<S, MODE>(p, sm, rq, gq, t, layer, q, tok, tg)) return;
+        if (!cls_qkv<S, MODE>(p, sm, rq, rq1, gq, t, layer, q, q1, tok, tg)) return;
         if constexpr (HAS_G) ld_gu<S>(rg, ru, gf, p, layer, gi, pace_units(p, PACE_QG_GU));
-        else if (has_next(p, t, layer)) ld_qkv<S>(rq, gq, p, next_layer(p, layer), q, pace_units(p, PACE_QG_Q));
+        else if (has_next(p, t, layer)) ld_qkv<S>(rq, rq1, gq, p, next_layer(p, layer), q, q1, pace_units(p, PACE_QG_Q));
       }
       if constexpr (HAS_G) {
         if (!cls_gu<S, MODE>(p, sm, rg, ru, gf, t, layer, gi, tg)) return;
         if (has_next(p, t, layer)) {
-          if constexpr (HAS_Q) ld_qkv<S>(rq, gq, p, next_layer(p, layer), q, pace_units(p, PACE_QG_Q));
+          if constexpr (HAS_Q) ld_qkv<S>(rq, rq1, gq, p, next_layer(p, layer), q, q1, pace_units(p, PACE_QG_Q));
           else ld_gu<S>(rg, ru, gf, p, next_layer(p, layer), gi, pace_units(p, PACE_QG_GU));
         }
       }
@@ -617,7 +635,7 @@ __device__ __forceinline__ void run_qg(const Params& p, Smem<S>& sm, const int* 
     LmWarm lw;
     lm_warm_load<S, MODE>(p, lw);
     if (!cls_lm_head<S, MODE>(p, sm, t, tb, [&]() {
-          if constexpr (HAS_Q) ld_qkv<S>(rq, gq, p, 0, q);
+          if constexpr (HAS_Q) ld_qkv<S>(rq, rq1, gq, p, 0, q, q1);
           else ld_gu<S>(rg, ru, gf, p, 0, gi);
         }, lw))
       return;
@@ -733,17 +751,27 @@ __global__ __launch_bounds__(NT) void decode_cls_kernel(Params p) {
   for (int i = threadIdx.x; i < NW * 16 * 32 * KVB; i += NT) (&sm.pb[0][0][0])[i] = 0;
   __syncthreads();
   const int* role = p.roles + blockIdx.x * ROLE_INTS;
-  switch (role[RF_CLS]) {
-    case CLS_ATT: run_att<S, MODE>(p, sm, role); break;
-    case CLS_A: run_att<S, MODE, false>(p, sm, role); break;
-    case CLS_QG: run_qg<S, MODE, true, true>(p, sm, role); break;
-    case CLS_Q: run_qg<S, MODE, true, false>(p, sm, role); break;
-    case CLS_G: run_qg<S, MODE, false, true>(p, sm, role); break;
-    case CLS_DG: run_down<S, MODE, CLS_DG>(p, sm, role); break;
-    case CLS_DO: run_down<S, MODE, CLS_DO>(p, sm, role); break;
-    case CLS_D: run_down<S, MODE, CLS_D>(p, sm, role); break;
-    case CLS_O: run_o<S, MODE>(p, sm, role); break;
-    default: run_idle<S, MODE>(p, sm); break;
+  if constexpr (S::Q_WG == 1) {
+    switch (role[RF_CLS]) {
+      case CLS_ATT: run_att<S, MODE>(p, sm, role); break;
+      case CLS_A: run_att<S, MODE, false>(p, sm, role); break;
+      case CLS_QG: run_qg<S, MODE, true, true>(p, sm, role); break;
+      case CLS_Q: run_qg<S, MODE, true, false>(p, sm, role); break;
+      case CLS_G: run_qg<S, MODE, false, true>(p, sm, role); break;
+      case CLS_DG: run_down<S, MODE, CLS_DG>(p, sm, role); break;
+      case CLS_DO: run_down<S, MODE, CLS_DO>(p, sm, role); break;
+      case CLS_D: run_down<S, MODE, CLS_D>(p, sm, role); break;
+      case CLS_O: run_o<S, MODE>(p, sm, role); break;
+      default: run_idle<S, MODE>(p, sm); break;
+    }
+  } else {  // the classes of such a shape's tables (build_roles)
+    switch (role[RF_CLS]) {
+      case CLS_A: run_att<S, MODE, false>(p, sm, role); break;
+      case CLS_QG: run_qg<S, MODE, true, true>(p, sm, role); break;
+      case CLS_DG: run_down<S, MODE, CLS_DG>(p, sm, role); break;
+      case CLS_O: run_o<S, MODE>(p, sm, role); break;
+      default: run_idle<S, MODE>(p, sm); break;
+    }
   }
   if (blockIdx.x == 0) {  // the last token's id
     const int t = p.n_tokens;

@@ -29,6 +29,9 @@ struct Shape {
   static constexpr int KC_Q = QD / 256;
   static constexpr int KC_F = F / 256;
   static constexpr int RB_QKV = QKV / 16;    // 16-row blocks of the fused QKV
+  // QKV blocks a workgroup of the class kernel takes: two where one each would
+  // leave too few of the 256 workgroups to the other roles
+  static constexpr int Q_WG = RB_QKV > 128 ? 2 : 1;
   static constexpr int RB_H = H / 16;        // 16-row blocks of O / down outputs
   static constexpr int RB_F = F / 16;        // 16-row blocks of gate (and of up)
   // Packed per-layer sizes in 16-byte units (one tile = 64 units = 1 KiB).

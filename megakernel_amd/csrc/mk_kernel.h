@@ -435,17 +435,20 @@ __device__ __forceinline__ float norm_scale(const float* ssw, float inv_h) {
 // the norm scale is taken here; its LDS reads issue with the shares' reads
 // (one round trip, not two).
 template <bool NORM = false>
+__device__ __forceinline__ void qkv_rows(const float* red, u64* dst16, float scale, unsigned tag, const float* ssw,
+                                         float inv_h, bool ok) {
+  const unsigned l = lane_id();
+  const float sh = red_row4(red, l);
+  const float s = NORM ? scale * norm_scale(ssw, inv_h) : scale;
+  const float y = sh * s;
+  if (ok && (l & 3u) == 0u) ll_put(dst16 + (l >> 2), ll_pack(y, tag));
+}
+template <bool NORM = false>
 __device__ __forceinline__ bool store_block(const float* red, u64* dst16, float scale, unsigned tag,
                                             const float* ssw = nullptr, float inv_h = 0.f) {
   __syncthreads();
   const bool ok = !block_aborted();  // read with the shares (one LDS round trip)
-  if (wave_id() == PUB_WAVE) {
-    const unsigned l = lane_id();
-    const float sh = red_row4(red, l);
-    const float s = NORM ? scale * norm_scale(ssw, inv_h) : scale;
-    const float y = sh * s;
-    if (ok && (l & 3u) == 0u) ll_put(dst16 + (l >> 2), ll_pack(y, tag));
-  }
+  if (wave_id() == PUB_WAVE) qkv_rows<NORM>(red, dst16, scale, tag, ssw, inv_h, ok);
   return ok;
 }
 
@@ -1381,8 +1384,9 @@ __device__ bool attention_merge(const Params& p, Smem<S>& sm, int g, int nsplit,
 // and merge them (log-sum-exp, reference attention.cuh:96-140 computes the
 // same softmax in one pass) into dst[QD], in batches of SB splits with a
 // running max; plus, unless xb0 < 0, the 16 residual rows of x block xb0
-// (threads 0..7) and, unless xb1 < 0, of block xb1 (threads 8..15).  Thread t
-// owns output pairs t + k NT (8-byte loads, as fetch_pk).  A batch's slots
+// (threads 0..7) and, unless xb1 < 0, of block xb1 (threads 8..15).  Each
+// thread owns one output pair per NT of them, wave w's together the
+// columns of its own O products (8-byte loads, as fetch_pk).  A batch's slots
 // past nsplit are skipped by wave-uniform branches; fetch_attn picks SB from
 // the split count, so the registers and the merge arithmetic of a round are
 // those of the splits that exist (the merge sits between the last poll round
@@ -1394,6 +1398,9 @@ __device__ __forceinline__ int fetch_attn_core(const Params& p, const u64* part,
   constexpr int WP = part_words<S>();
   constexpr int PPT = (S::QD / 2 + NT - 1) / NT;
   const int tid = ltid();
+  const auto pair_of = [tid](int k) {
+    return S::QD / 2 % NT == 0 ? tid / kWave * (PPT * kWave) + k * kWave + tid % kWave : tid + k * NT;
+  };
   const bool want_x0 = xb0 >= 0 && (tid < 8 || (tid < 16 && xb1 >= 0));
   int failed = 0;
   float M[PPT], L[PPT], o0[PPT], o1[PPT];
@@ -1408,7 +1415,7 @@ __device__ __forceinline__ int fetch_attn_core(const Params& p, const u64* part,
     while (true) {
 #pragma unroll
       for (int k = 0; k < PPT; ++k) {
-        const int pi = tid + k * NT < S::QD / 2 ? tid + k * NT : 0;
+        const int pi = pair_of(k) < S::QD / 2 ? pair_of(k) : 0;
         const int g = pi / NPG, pg = pi % NPG, j = (2 * pg) / S::D;
 #pragma unroll
         for (int u = 0; u < SB; ++u) {
@@ -1426,7 +1433,7 @@ __device__ __forceinline__ int fetch_attn_core(const Params& p, const u64* part,
       for (int k = 0; k < PPT; ++k)
 #pragma unroll
         for (int u = 0; u < SB; ++u)
-          ready &= tid + k * NT >= S::QD / 2 || s0 + u >= nsplit ||
+          ready &= pair_of(k) >= S::QD / 2 || s0 + u >= nsplit ||
                    (pk_ready(wa[k][u], t4) && pk_ready(wm[k][u], t4));
       if (ready) break;
       if (!sp.step(p.err, p.timeout_ticks)) {
@@ -1460,7 +1467,7 @@ __device__ __forceinline__ int fetch_attn_core(const Params& p, const u64* part,
   }
 #pragma unroll
   for (int k = 0; k < PPT; ++k) {
-    const int pi = tid + k * NT;
+    const int pi = pair_of(k);
     if (pi < S::QD / 2) {
       const float il = __builtin_amdgcn_rcpf(L[k]);  // one reciprocal (~1 ulp) for both outputs
       xs_put_pair(reinterpret_cast<uint32_t*>(dst), 2 * pi, o0[k] * il, o1[k] * il);
@@ -1496,9 +1503,9 @@ __device__ __forceinline__ bool fetch_attn(const Params& p, const u64* part, int
   return !block_failed(fetch_attn_any<S>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev));
 }
 
-// Barrier-free form (class kernel).  When the pairs are as many as the
-// threads (BASELINE: QD / 2 = 512), thread t stages pair t, so wave w stages
-// exactly the QD / NW input columns its own block products read (LDS
+// Barrier-free form (class kernel).  When the pairs are whole rounds of the
+// threads (QD / 2 = 512 or 1,024), wave w stages exactly the QD / NW input
+// columns its own block products read (LDS
 // operations of one wave complete in order): no barrier before the products.
 // No barrier before the wait either: every LDS word this phase writes (its
 // staged input, block shares, residual rows) was last read in this
@@ -1511,7 +1518,7 @@ __device__ __forceinline__ void fetch_attn_nb(const Params& p, const u64* part, 
                                               int xb0, int xb1, unsigned xt4, float* dst, float* xres,
                                               EvPoll ev = EvPoll()) {
   if (fetch_attn_any<S>(p, part, nsplit, t4, x, xb0, xb1, xt4, dst, xres, ev)) wg_abort = 1;
-  if constexpr (S::QD / 2 != NT) __syncthreads();  // a wave's pairs are not its own input columns
+  if constexpr (S::QD / 2 % NT != 0) __syncthreads();  // a wave's pairs are not its own input columns
   else asm volatile("" ::: "memory");              // staging stores before the wave's B-operand reads
 }
 

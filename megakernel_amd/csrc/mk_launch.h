@@ -37,13 +37,15 @@ static void launch_cls(int grid, hipStream_t stream, const Params& p) {
   hipLaunchKernelGGL((decode_cls_kernel<S, MODE>), dim3(grid), dim3(NT), 0, stream, p);
 }
 
-template <class S, bool HAS_CLS>
+// HAS_CLS / HAS_W8: the shape has class-kernel instantiations, and those with
+// FP8 layer weights.
+template <class S, bool HAS_CLS, bool HAS_W8 = HAS_CLS>
 static hipError_t launch_decode(int grid, hipStream_t stream, const Params& p, bool lc, bool cls) {
   const int mode = (lc ? 1 : 0) | (p.trace || p.dbg_layers || p.dbg_logits ? 2 : 0) | (p.lmhead8 ? 4 : 0) |
                    (p.kscale ? 8 : 0);
   if constexpr (HAS_CLS) {
-    if (cls && !lc) {
-      switch (mode | (p.layers8 ? 16 : 0)) {
+    if (cls && !lc && !p.layers8) {
+      switch (mode) {
         case 0: launch_cls<S, 0>(grid, stream, p); break;
         case 2: launch_cls<S, 2>(grid, stream, p); break;
         case 4: launch_cls<S, 4>(grid, stream, p); break;
@@ -51,17 +53,24 @@ static hipError_t launch_decode(int grid, hipStream_t stream, const Params& p, b
         case 8: launch_cls<S, 8>(grid, stream, p); break;
         case 10: launch_cls<S, 10>(grid, stream, p); break;
         case 12: launch_cls<S, 12>(grid, stream, p); break;
-        case 14: launch_cls<S, 14>(grid, stream, p); break;
-        case 16: launch_cls<S, 16>(grid, stream, p); break;
-        case 18: launch_cls<S, 18>(grid, stream, p); break;
-        case 20: launch_cls<S, 20>(grid, stream, p); break;
-        case 22: launch_cls<S, 22>(grid, stream, p); break;
-        case 24: launch_cls<S, 24>(grid, stream, p); break;
-        case 26: launch_cls<S, 26>(grid, stream, p); break;
-        case 28: launch_cls<S, 28>(grid, stream, p); break;
-        default: launch_cls<S, 30>(grid, stream, p); break;
+        default: launch_cls<S, 14>(grid, stream, p); break;
       }
       return hipGetLastError();
+    }
+    if constexpr (HAS_W8) {
+      if (cls && !lc) {
+        switch (mode) {
+          case 0: launch_cls<S, 16>(grid, stream, p); break;
+          case 2: launch_cls<S, 18>(grid, stream, p); break;
+          case 4: launch_cls<S, 20>(grid, stream, p); break;
+          case 6: launch_cls<S, 22>(grid, stream, p); break;
+          case 8: launch_cls<S, 24>(grid, stream, p); break;
+          case 10: launch_cls<S, 26>(grid, stream, p); break;
+          case 12: launch_cls<S, 28>(grid, stream, p); break;
+          default: launch_cls<S, 30>(grid, stream, p); break;
+        }
+        return hipGetLastError();
+      }
     }
   }
   if (p.layers8) return hipErrorInvalidValue;  // the spread kernel reads bf16 layer weights only
@@ -100,7 +109,7 @@ static int occupancy_cls() {
   return n;
 }
 
-template <class S, bool HAS_CLS>
+template <class S, bool HAS_CLS, bool HAS_W8 = HAS_CLS>
 static int occupancy_min() {
   const int n[16] = {occupancy_of<S, 0>(),  occupancy_of<S, 1>(),  occupancy_of<S, 2>(),  occupancy_of<S, 3>(),
                      occupancy_of<S, 4>(),  occupancy_of<S, 5>(),  occupancy_of<S, 6>(),  occupancy_of<S, 7>(),
@@ -109,11 +118,14 @@ static int occupancy_min() {
   int m = n[0];
   for (int i = 1; i < 16; ++i) m = n[i] < m ? n[i] : m;
   if constexpr (HAS_CLS) {
-    const int c[16] = {occupancy_cls<S, 0>(),  occupancy_cls<S, 2>(),  occupancy_cls<S, 4>(),  occupancy_cls<S, 6>(),
-                       occupancy_cls<S, 8>(),  occupancy_cls<S, 10>(), occupancy_cls<S, 12>(), occupancy_cls<S, 14>(),
-                       occupancy_cls<S, 16>(), occupancy_cls<S, 18>(), occupancy_cls<S, 20>(), occupancy_cls<S, 22>(),
-                       occupancy_cls<S, 24>(), occupancy_cls<S, 26>(), occupancy_cls<S, 28>(), occupancy_cls<S, 30>()};
-    for (int i = 0; i < 16; ++i) m = c[i] < m ? c[i] : m;
+    const int c[8] = {occupancy_cls<S, 0>(), occupancy_cls<S, 2>(),  occupancy_cls<S, 4>(),  occupancy_cls<S, 6>(),
+                      occupancy_cls<S, 8>(), occupancy_cls<S, 10>(), occupancy_cls<S, 12>(), occupancy_cls<S, 14>()};
+    for (int i = 0; i < 8; ++i) m = c[i] < m ? c[i] : m;
+  }
+  if constexpr (HAS_W8) {
+    const int c[8] = {occupancy_cls<S, 16>(), occupancy_cls<S, 18>(), occupancy_cls<S, 20>(), occupancy_cls<S, 22>(),
+                      occupancy_cls<S, 24>(), occupancy_cls<S, 26>(), occupancy_cls<S, 28>(), occupancy_cls<S, 30>()};
+    for (int i = 0; i < 8; ++i) m = c[i] < m ? c[i] : m;
   }
   return m;
 }

@@ -556,3 +556,35 @@ def test_resident_launch_opens_an_attention_split():
     finally:
         eng.close()
         dw.free()
+
+
+@pytest.mark.parametrize("ctx", [1, 255, 700, 1016, 1300, 1530, 1600])
+def test_qwen3_class_kernel_equals_spread(ctx):
+    """head_dim 128: the class kernel (two QKV blocks per workgroup, one to
+    four splits, widened ones up to 384 positions) against the spread kernel
+    on the same cache: the same sums in other splits, so equal to the packed
+    partials' 2^-20 rounding carried through four layers; resident == per token
+    (1,530 ends in the class kernel's range, 1,600 past it)."""
+    shape = QWEN3_06B.with_(n_layers=4, vocab=4096)
+    dw = DeviceWeights(shape, 31, gain_std=0.1)
+    eng = MegakernelEngine(shape=shape, max_seq=2048, device_weights=dw)
+    try:
+        eng.fill_kv_synthetic(ctx, 9)
+        assert eng.decode_kernel_for(6) == (_lib.KERNEL_SPREAD if ctx > 1536 else _lib.KERNEL_CLASS)
+        got = eng.decode_many(5, 5)
+        nxt, layers, logits = eng.debug_forward(got[-1])
+        eng.set_pos(ctx)
+        tok, want = 5, []
+        for _ in range(5):
+            tok = eng.decode_token(tok)
+            want.append(tok)
+        assert got == want
+        eng.set_decode_kernel(_lib.KERNEL_SPREAD)
+        eng.set_pos(ctx)
+        assert eng.decode_many(5, 5) == got
+        nxt_s, layers_s, logits_s = eng.debug_forward(got[-1])
+        assert nxt_s == nxt
+        assert rel_l2(layers, layers_s).max() < 1e-4 and rel_l2(logits, logits_s) < 1e-4
+    finally:
+        eng.close()
+        dw.free()
