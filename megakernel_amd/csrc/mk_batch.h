@@ -88,13 +88,13 @@ struct BParams {
   int s_pad;
   // activations, per slot (x_slot .. act_slot below: L + 1 slots of x / xg /
   // ssq, L of qkv / att / act; the per-phase kernels use slot 0)
-  float* x;                 // [slot][2 consumers][BMAX][H] residual streams
-  uint16_t* xg;             // [slot][2 consumers][2 planes][BMAX][H] x * gain as bf16 hi / lo parts:
+  float* x;                 // [slot][2 consumers][H/16][BMAX][16] residual streams (x_at)
+  uint16_t* xg;             // [slot][2 consumers][2 planes][H/32][64][8] x * gain as bf16 hi / lo parts (unit_at):
                             //   consumer 0 = attn_norm of the next QKV (or final_norm), 1 = ffn_norm
   float* ssq;               // [slot][2 consumers][H/16][BMAX] sums of squares of x per 16-row block
   float* qkv;               // [slot][BMAX][QKV] raw projections
-  uint16_t* att;            // [slot][2][BMAX][QD] merged attention output, bf16 hi / lo parts
-  uint16_t* act;            // [slot][2][BMAX][F] SiLU(g) * u, bf16 hi / lo parts
+  uint16_t* att;            // [slot][2][QD/32][64][8] merged attention output, bf16 hi / lo parts
+  uint16_t* act;            // [slot][2][F/32][64][8] SiLU(g) * u, bf16 hi / lo parts
   float* part;              // [BMAX][NKV][nsplit_max][PW] attention partials
   int* cnt;                 // [BMAX][NKV] finished splits of the current layer
   float* gpart;             // split-K partial block sums of the GEMM kernels
@@ -225,6 +225,23 @@ __device__ __forceinline__ uint16_t* act_slot(const BParams& p, int slot) {
   return p.act + (long long)slot * 2 * BMAX * S::F;
 }
 
+// Layouts of the activations inside a slot (K columns, up to 16 sequences or
+// tokens n).  The bf16 planes that feed a product (xg, att, act) are stored as
+// its B operand: 1 KiB units of 32 k's, lane (k / 8 % 4) * 16 + n holding 8
+// consecutive k's of column n, so a wave loads a unit with one contiguous
+// 16-byte load per lane and an epilogue lane, which holds four rows of one
+// column, stores 8 bytes.  (Row-major planes cost a load instruction 16 lines
+// at a 2 KiB stride and an epilogue four 2-byte stores per plane.  With units a
+// 1,024-token prefill went from 4.02 to 3.41 ms -- gate / up 39 -> 34, down 32
+// -> 24, O 19 -> 12 us per layer -- and a batched step's QKV, O, gate / up and
+// down from 5.0, 5.5, 6.6 and 7.2 to 4.6, 4.8, 5.1 and 6.3 us.)  The fp32 residual stream holds the
+// 16 rows of a block per column, one 16-byte access per epilogue lane.
+__device__ __forceinline__ int unit_at(int n, int k) { return ((k >> 5) * 64 + ((k >> 3) & 3) * 16 + n) * 8 + (k & 7); }
+__device__ __forceinline__ void st4(uint16_t* a, const uint16_t (&v)[4]) {
+  *reinterpret_cast<u32x2*>(a) = u32x2{v[0] | (unsigned)v[1] << 16, v[2] | (unsigned)v[3] << 16};
+}
+__device__ __forceinline__ int x_at(int n, int row) { return ((row >> 4) * BMAX + n) * 16 + (row & 15); }
+
 // Epilogue of an x-producing 16-row block: thread t < 256 holds the new x of
 // row rb * 16 + t / 16, sequence t % 16.  red: >= 256 floats of LDS.
 // Stores of activations handed between workgroups: ordinary between kernels
@@ -243,11 +260,11 @@ __device__ __forceinline__ void publish_x(const BParams& p, int slot, int c, con
   if (t < 256) {
     const bool on = b < p.B;
     if (on) {
-      st_act<SC1>(x_slot<S>(p, slot, c) + (long long)b * S::H + row, xn);
+      st_act<SC1>(x_slot<S>(p, slot, c) + x_at(b, row), xn);
       uint16_t h, o;
       split2(xn * bf16_to_f32(gain[row]), h, o);
-      st_act<SC1>(xg_plane<S>(p, slot, c, 0) + (long long)b * S::H + row, h);
-      st_act<SC1>(xg_plane<S>(p, slot, c, 1) + (long long)b * S::H + row, o);
+      st_act<SC1>(xg_plane<S>(p, slot, c, 0) + unit_at(b, row), h);
+      st_act<SC1>(xg_plane<S>(p, slot, c, 1) + unit_at(b, row), o);
     }
     red[t] = on ? xn * xn : 0.f;
   }
@@ -308,24 +325,22 @@ __device__ __forceinline__ void load_tiles(ATiles<NT>& a, const u32x4* __restric
     a.t[j] = w + GW * j < NT ? buf_ld_nt(rs, l * 16u, (unsigned)(kt0 + w + GW * j) * 1024u) : u32x4{0u, 0u, 0u, 0u};
 }
 
-// The 16 activation columns of this wave's tiles: the B operands.  Planes:
-// element (n, k) at hi[n * ld + k], lo[n * ld + k].  Loaded on their own, so
+// The 16 activation columns of this wave's tiles: the B operands, from the
+// planes' units (unit_at).  Loaded on their own, so
 // a block can issue its other loads (norm sums, residual) before it waits.
 template <int NT>
 struct BCols {
   u32x4 h[ATiles<NT>::TW], l[ATiles<NT>::TW];
 };
 template <int NT>
-__device__ __forceinline__ void load_cols(BCols<NT>& c, const uint16_t* hi, const uint16_t* lo, int ld, int kt0) {
-  const unsigned l = lane_id();
-  const int w = wave_id();
-  const int bo = (int)(l & 15u) * ld + 8 * (int)(l >> 4);
+__device__ __forceinline__ void load_cols(BCols<NT>& c, const uint16_t* hi, const uint16_t* lo, int kt0) {
+  const int w = wave_id(), bo = 8 * (int)lane_id();
 #pragma unroll
   for (int j = 0; j < ATiles<NT>::TW; ++j) {
     const int kt = kt0 + w + GW * j;
     if (w + GW * j < NT) {
-      c.h[j] = *reinterpret_cast<const u32x4*>(hi + bo + 32 * kt);
-      c.l[j] = *reinterpret_cast<const u32x4*>(lo + bo + 32 * kt);
+      c.h[j] = *reinterpret_cast<const u32x4*>(hi + bo + 512 * kt);
+      c.l[j] = *reinterpret_cast<const u32x4*>(lo + bo + 512 * kt);
     }
   }
 }
@@ -441,11 +456,11 @@ __global__ __launch_bounds__(256) void bk_embed(G pg) {
     const float xv = on ? bf16_to_f32(u[e]) : 0.f;
     xs[k] = xv;
     if (on) {
-      x_slot<S>(p, 0, 0)[(long long)b * S::H + k] = xv;
+      x_slot<S>(p, 0, 0)[x_at(b, k)] = xv;
       uint16_t h, o;
       split2(xv * bf16_to_f32(p.norms[S::NORM_ATTN + k]), h, o);
-      xg_plane<S>(p, 0, 0, 0)[(long long)b * S::H + k] = h;
-      xg_plane<S>(p, 0, 0, 1)[(long long)b * S::H + k] = o;
+      xg_plane<S>(p, 0, 0, 0)[unit_at(b, k)] = h;
+      xg_plane<S>(p, 0, 0, 1)[unit_at(b, k)] = o;
     }
   }
   __syncthreads();
@@ -524,7 +539,7 @@ __device__ __forceinline__ bool qkv_block(const BParams& p, int layer, int ep, i
   if (!ready()) return false;
   const int sl = FUSED ? layer : 0;
   BCols<NT> c;
-  load_cols(c, xg_plane<S>(p, sl, 0, 0), xg_plane<S>(p, sl, 0, 1), S::H, kt0);
+  load_cols(c, xg_plane<S>(p, sl, 0, 0), xg_plane<S>(p, sl, 0, 1), kt0);
   rnorm<S>(p, sl, 0, rr);
   float v[1] = {block_reduce(tiles_mma(a, c), red)};
   if (!splitk_finish(p, rb, ks, KS_QKV, v, last)) return true;
@@ -546,9 +561,9 @@ __device__ __forceinline__ bool o_block(const BParams& p, int layer, int ep, int
   const int sl = FUSED ? layer : 0;
   const uint16_t* at = att_slot<S>(p, sl);
   BCols<NT> c;
-  load_cols(c, at, at + BMAX * S::QD, S::QD, kt0);
+  load_cols(c, at, at + BMAX * S::QD, kt0);
   const int t = ltid(), b = t % 16;
-  const float xin = t < 256 && b < p.B ? x_slot<S>(p, sl, 0)[(long long)b * S::H + rb * 16 + t / 16] : 0.f;
+  const float xin = t < 256 && b < p.B ? x_slot<S>(p, sl, 0)[x_at(b, rb * 16 + t / 16)] : 0.f;
   float v[1] = {block_reduce(tiles_mma(a, c), red)};
   if (!splitk_finish(p, rb, ks, KS_O, v, last)) return true;
   const float xn = t < 256 && b < p.B ? xin + v[0] : 0.f;
@@ -571,7 +586,7 @@ __device__ __forceinline__ bool gu_block(const BParams& p, int layer, int ep, in
   if (!ready()) return false;
   const int sl = FUSED ? layer : 0;
   BCols<NT> c;
-  load_cols(c, xg_plane<S>(p, sl, 1, 0), xg_plane<S>(p, sl, 1, 1), S::H, kt0);
+  load_cols(c, xg_plane<S>(p, sl, 1, 0), xg_plane<S>(p, sl, 1, 1), kt0);
   rnorm<S>(p, sl, 1, rr);
   f32x4 pg, pu;
   tiles_mma2(ag, au, c, pg, pu);
@@ -585,8 +600,8 @@ __device__ __forceinline__ bool gu_block(const BParams& p, int layer, int ep, in
     const float g = v[0] * rr[b], u = v[1] * rr[b];
     uint16_t h, o;
     split2(g / (1.0f + __expf(-g)) * u, h, o);  // SiLU(g) * u (reference utils.cuh:59-61)
-    st_act<FUSED>(act_slot<S>(p, sl) + (long long)b * S::F + row, h);
-    st_act<FUSED>(act_slot<S>(p, sl) + (long long)(BMAX + b) * S::F + row, o);
+    st_act<FUSED>(act_slot<S>(p, sl) + unit_at(b, row), h);
+    st_act<FUSED>(act_slot<S>(p, sl) + BMAX * S::F + unit_at(b, row), o);
   }
   if constexpr (FUSED) fc_done(p, layer, FC_GU, rb, ep);
   return true;
@@ -606,12 +621,12 @@ __device__ __forceinline__ bool down_block(const BParams& p, int layer, int ep, 
   const int sl = FUSED ? layer : 0;
   const uint16_t* ac = act_slot<S>(p, sl);
   BCols<NT> c;
-  load_cols(c, ac, ac + BMAX * S::F, S::F, kt0);
+  load_cols(c, ac, ac + BMAX * S::F, kt0);
   const int t = ltid(), b = t % 16;
   // the residual, read by the workgroup that finishes the block (split 0 in
   // the one-kernel step, whichever split completes it otherwise)
   const float xin = (!FUSED || ks == 0) && t < 256 && b < p.B
-                        ? x_slot<S>(p, sl, 1)[(long long)b * S::H + rb * 16 + t / 16]
+                        ? x_slot<S>(p, sl, 1)[x_at(b, rb * 16 + t / 16)]
                         : 0.f;
   float v[1] = {block_reduce(tiles_mma(a, c), red)};
   if constexpr (FUSED) {
@@ -836,8 +851,8 @@ __global__ __launch_bounds__(GT) void bk_pgu_t(PGroup pg, int layer) {
       const int kt = (i / kWave) % KC, ln = i % kWave;
       xb[k] = u32x4{0u, 0u, 0u, 0u};
       if (gq < ngr)
-        xb[k] = *reinterpret_cast<const u32x4*>(xg_plane<S>(group_params(pg, g0 + gq), 0, 1, pl) + (ln & 15) * S::H +
-                                                 32 * (c * KC + kt) + 8 * (ln >> 4));
+        xb[k] = *reinterpret_cast<const u32x4*>(xg_plane<S>(group_params(pg, g0 + gq), 0, 1, pl) +
+                                                 512 * (c * KC + kt) + 8 * ln);
     }
   };
   const auto store = [&](int buf, const u32x4(&xa)[LA], const u32x4(&xb)[LB]) {
@@ -858,8 +873,7 @@ __global__ __launch_bounds__(GT) void bk_pgu_t(PGroup pg, int layer) {
     for (int k = 0; k < LB; ++k) {
       const int t = w + GW * k, gq = t / (2 * KC), pl = (t / KC) % 2, kt = t % KC;
       const int gs = gq < ngr ? gq : 0;  // a group past the pass reads group 0 (its columns are never stored)
-      lds_load16(xg_plane<S>(group_params(pg, g0 + gs), 0, 1, pl) + (ln & 15) * S::H + 32 * (c * KC + kt) +
-                     8 * (ln >> 4),
+      lds_load16(xg_plane<S>(group_params(pg, g0 + gs), 0, 1, pl) + 512 * (c * KC + kt) + 8 * ln,
                  &sb[buf][gq][pl][kt][0]);
     }
   };
@@ -936,17 +950,18 @@ __global__ __launch_bounds__(GT) void bk_pgu_t(PGroup pg, int layer) {
     const float rs = rsqrtf(ss / (float)S::H + kRmsEps);
     if (n < p.B) {
 #pragma unroll
-      for (int r = 0; r < WB; ++r)
+      for (int r = 0; r < WB; ++r) {
+        uint16_t h[4], o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int row = (rb0 + pw + r) * 16 + 4 * kg + i;
           const float g = (acc[r][j][0][0][i] + acc[r][j][0][1][i]) * rs;
           const float u = (acc[r][j][1][0][i] + acc[r][j][1][1][i]) * rs;
-          uint16_t h, o;
-          split2(g / (1.0f + __expf(-g)) * u, h, o);  // SiLU(g) * u (reference utils.cuh:59-61)
-          act_slot<S>(p, 0)[(long long)n * S::F + row] = h;
-          act_slot<S>(p, 0)[(long long)(BMAX + n) * S::F + row] = o;
+          split2(g / (1.0f + __expf(-g)) * u, h[i], o[i]);  // SiLU(g) * u (reference utils.cuh:59-61)
         }
+        uint16_t* a = act_slot<S>(p, 0) + unit_at(n, (rb0 + pw + r) * 16 + 4 * kg);
+        st4(a, h);
+        st4(a + BMAX * S::F, o);
+      }
     }
   }
 }
@@ -991,8 +1006,7 @@ __global__ __launch_bounds__(GT) void bk_ptile(PGroup pg, int layer) {
       const int kt = (i / kWave) % KC, ln = i % kWave;
       xb[k] = u32x4{0u, 0u, 0u, 0u};
       if (gq < ngr)
-        xb[k] = *reinterpret_cast<const u32x4*>(plane(group_params(pg, g0 + gq), pl) + (ln & 15) * K +
-                                                 32 * (c * KC + kt) + 8 * (ln >> 4));
+        xb[k] = *reinterpret_cast<const u32x4*>(plane(group_params(pg, g0 + gq), pl) + 512 * (c * KC + kt) + 8 * ln);
     }
   };
   const auto store = [&](int buf, const u32x4(&xa)[LA], const u32x4(&xb)[LB]) {
@@ -1013,8 +1027,7 @@ __global__ __launch_bounds__(GT) void bk_ptile(PGroup pg, int layer) {
     for (int k = 0; k < LB; ++k) {
       const int t = w + GW * k, gq = t / (2 * KC), pl = (t / KC) % 2, kt = t % KC;
       const int gs = gq < ngr ? gq : 0;  // a group past the pass reads group 0 (its columns are never stored)
-      lds_load16(plane(group_params(pg, g0 + gs), pl) + (ln & 15) * K + 32 * (c * KC + kt) + 8 * (ln >> 4),
-                 &sb[buf][gq][pl][kt][0]);
+      lds_load16(plane(group_params(pg, g0 + gs), pl) + 512 * (c * KC + kt) + 8 * ln, &sb[buf][gq][pl][kt][0]);
     }
   };
   if constexpr (T::NS == 0) {
@@ -1088,10 +1101,8 @@ __global__ __launch_bounds__(GT) void bk_ptile(PGroup pg, int layer) {
       if (on) {
 #pragma unroll
         for (int r = 0; r < WB; ++r)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            qkv_slot<S>(p, 0)[(long long)n * S::QKV + (rb0 + pw + r) * 16 + 4 * kg + i] =
-                (acc[r][j][0][i] + acc[r][j][1][i]) * rs;
+          *reinterpret_cast<f32x4*>(qkv_slot<S>(p, 0) + (long long)n * S::QKV + (rb0 + pw + r) * 16 + 4 * kg) =
+              (acc[r][j][0] + acc[r][j][1]) * rs;
       }
     } else {
       // O: residual stream copy 0 in, copy 1 + the FFN norm's parts out;
@@ -1105,20 +1116,23 @@ __global__ __launch_bounds__(GT) void bk_ptile(PGroup pg, int layer) {
       for (int r = 0; r < WB; ++r) {
         const int rb = rb0 + pw + r;
         float sq = 0.f;
+        const int row = rb * 16 + 4 * kg;
+        f32x4 xn = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (on) {
+          xn = *reinterpret_cast<const f32x4*>(x_slot<S>(p, 0, CI) + x_at(n, row));
+          const u32x2 gw = *reinterpret_cast<const u32x2*>(gain + row);
+          uint16_t h[4], o[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int row = rb * 16 + 4 * kg + i;
-          const long long e = (long long)n * S::H + row;
-          const float xn = on ? x_slot<S>(p, 0, CI)[e] + (acc[r][j][0][i] + acc[r][j][1][i]) : 0.f;
-          if (on) {
-            x_slot<S>(p, 0, CO)[e] = xn;
-            uint16_t h, o;
-            split2(xn * bf16_to_f32(gain[row]), h, o);
-            xg_plane<S>(p, 0, CO, 0)[e] = h;
-            xg_plane<S>(p, 0, CO, 1)[e] = o;
+          for (int i = 0; i < 4; ++i) {
+            xn[i] += acc[r][j][0][i] + acc[r][j][1][i];
+            split2(xn[i] * bf16_to_f32((uint16_t)(gw[i / 2] >> (16 * (i & 1)))), h[i], o[i]);
           }
-          sq += xn * xn;
+          *reinterpret_cast<f32x4*>(x_slot<S>(p, 0, CO) + x_at(n, row)) = xn;
+          st4(xg_plane<S>(p, 0, CO, 0) + unit_at(n, row), h);
+          st4(xg_plane<S>(p, 0, CO, 1) + unit_at(n, row), o);
         }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sq += xn[i] * xn[i];
         sq = sum_xor32(sum_xor16(sq));
         if (kg == 0) ssq_slot<S>(p, 0, CO)[(long long)rb * BMAX + n] = sq;
       }
@@ -1135,16 +1149,14 @@ __global__ __launch_bounds__(GT) void bk_lm(BParams p, int slot) {
   // F8: the FP8 copy; a lane's 16 bytes (row l & 15, columns 64 u + 16 kg ..
   // + 15 of unit u) feed two MFMA k-steps, whose B operands take the same
   // columns of the hidden state; the row scale enters the conversion
-  constexpr int LD = S::H + 8;  // padded LDS rows: the 16 sequences on different banks
-  __shared__ __attribute__((aligned(16))) uint16_t hi[BMAX * LD], lo[BMAX * LD];
+  __shared__ __attribute__((aligned(16))) uint16_t hi[BMAX * S::H], lo[BMAX * S::H];  // B-operand units (unit_at)
   __shared__ u64 best_w[GW][BMAX];
   __shared__ float rr[RR_N];
   {  // the final-norm parts published by the last layer, copied to LDS
     const uint16_t *gh = xg_plane<S>(p, slot, 0, 0), *gl = xg_plane<S>(p, slot, 0, 1);
     for (int i = threadIdx.x; i < BMAX * S::H / 8; i += GT) {
-      const int b = i / (S::H / 8), k = (i % (S::H / 8)) * 8;
-      *reinterpret_cast<u32x4*>(hi + b * LD + k) = *reinterpret_cast<const u32x4*>(gh + (long long)b * S::H + k);
-      *reinterpret_cast<u32x4*>(lo + b * LD + k) = *reinterpret_cast<const u32x4*>(gl + (long long)b * S::H + k);
+      reinterpret_cast<u32x4*>(hi)[i] = reinterpret_cast<const u32x4*>(gh)[i];
+      reinterpret_cast<u32x4*>(lo)[i] = reinterpret_cast<const u32x4*>(gl)[i];
     }
     rnorm<S>(p, slot, 0, rr);
   }
@@ -1153,7 +1165,7 @@ __global__ __launch_bounds__(GT) void bk_lm(BParams p, int slot) {
   const int w = wave_id();
   const int n = (int)(l & 15u), kg = (int)(l >> 4);
   const int nb = p.V / 16;
-  const int bo = n * LD + 8 * kg;
+  const int bo = 8 * (int)l;
   const float rn = rr[n];
   u64 best = 0ull;
   // the wave's blocks rb0, rb0 + stride, ... as a flat sequence of chunks of
@@ -1184,17 +1196,17 @@ __global__ __launch_bounds__(GT) void bk_lm(BParams p, int slot) {
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
           const u32x4 wb = fp8x8_to_bf16x8_scaled(half ? u32x2{cur[u][2], cur[u][3]} : u32x2{cur[u][0], cur[u][1]}, sc);
-          const int col = 64 * kt + 16 * kg + 8 * half - 8 * kg;  // bo already holds 8 kg
-          a0 = mfma(wb, *reinterpret_cast<const u32x4*>(hi + bo + col), a0);
-          a1 = mfma(wb, *reinterpret_cast<const u32x4*>(lo + bo + col), a1);
+          const int at = unit_at(n, 64 * kt + 16 * kg + 8 * half);
+          a0 = mfma(wb, *reinterpret_cast<const u32x4*>(hi + at), a0);
+          a1 = mfma(wb, *reinterpret_cast<const u32x4*>(lo + at), a1);
         }
       }
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int kt = k0 + u;
-        a0 = mfma(cur[u], *reinterpret_cast<const u32x4*>(hi + bo + 32 * kt), a0);
-        a1 = mfma(cur[u], *reinterpret_cast<const u32x4*>(lo + bo + 32 * kt), a1);
+        a0 = mfma(cur[u], *reinterpret_cast<const u32x4*>(hi + bo + 512 * kt), a0);
+        a1 = mfma(cur[u], *reinterpret_cast<const u32x4*>(lo + bo + 512 * kt), a1);
       }
     }
     if (c % CPB == CPB - 1) {  // the block is complete
@@ -1645,9 +1657,9 @@ __device__ __forceinline__ bool attn_item(const BParams& p, int layer, int ep, A
       }
       uint16_t hi, lo;
       split2(oo / ll, hi, lo);
-      const long long k = (long long)b * S::QD + g * 2 * D + tid;
+      const int k = unit_at(b, g * 2 * D + tid);
       st_act<FUSED>(att_slot<S>(p, sl) + k, hi);
-      st_act<FUSED>(att_slot<S>(p, sl) + (long long)BMAX * S::QD + k, lo);
+      st_act<FUSED>(att_slot<S>(p, sl) + BMAX * S::QD + k, lo);
     }
   }
   if constexpr (FUSED) {  // the merged output is acknowledged before it is counted
@@ -1968,28 +1980,34 @@ __global__ __launch_bounds__(PC_AW * kWave) void bk_pattn(PGroup pg, int layer) 
     }
   }
   __syncthreads();
-  {
-    const int d = tid % D;
+  {  // thread: 8 dims of one query, one 16-byte store per plane
+    static_assert(NT * 8 == PC_NQ * D, "eight outputs per thread");
+    const int q = tid / (D / 8), d0 = tid % (D / 8) * 8, col = q >> 1, j = q & 1;
+    if (col >= p.B) return;
+    float M = mw[0][q];
 #pragma unroll
-    for (int k = 0; k < PC_NQ / (NT / D); ++k) {
-      const int q = tid / D + (NT / D) * k, col = q >> 1, j = q & 1;
-      if (col >= p.B) continue;
-      float M = mw[0][q];
+    for (int i = 1; i < AWc; ++i) M = fmaxf(M, mw[i][q]);
+    float o[8], L = 0.f;
 #pragma unroll
-      for (int i = 1; i < AWc; ++i) M = fmaxf(M, mw[i][q]);
-      float o = 0.f, L = 0.f;
+    for (int e = 0; e < 8; ++e) o[e] = 0.f;
 #pragma unroll
-      for (int i = 0; i < AWc; ++i) {
-        const float f = mw[i][q] == -INFINITY ? 0.f : exp2f(mw[i][q] - M);
-        o = fmaf(f, ow[i][q][d], o);
-        L = fmaf(f, lw[i][q], L);
-      }
-      uint16_t hi, lo;
-      split2(o / L, hi, lo);
-      const long long k0 = (long long)col * S::QD + (g * 2 + j) * D + d;
-      att_slot<S>(p, 0)[k0] = hi;
-      att_slot<S>(p, 0)[(long long)BMAX * S::QD + k0] = lo;
+    for (int i = 0; i < AWc; ++i) {
+      const float f = mw[i][q] == -INFINITY ? 0.f : exp2f(mw[i][q] - M);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = fmaf(f, ow[i][q][d0 + e], o[e]);
+      L = fmaf(f, lw[i][q], L);
     }
+    u32x4 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint16_t h0, l0, h1, l1;
+      split2(o[2 * e] / L, h0, l0);
+      split2(o[2 * e + 1] / L, h1, l1);
+      hi[e] = h0 | (unsigned)h1 << 16, lo[e] = l0 | (unsigned)l1 << 16;
+    }
+    uint16_t* a = att_slot<S>(p, 0) + unit_at(col, (g * 2 + j) * D + d0);
+    *reinterpret_cast<u32x4*>(a) = hi;
+    *reinterpret_cast<u32x4*>(a + BMAX * S::QD) = lo;
   }
 }
 
