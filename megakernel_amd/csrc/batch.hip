@@ -117,25 +117,73 @@ static int launch_step(BHandle* h, const BParams& p) {
   return 0;
 }
 
+// One GEMM of a prefill pass (bk_pgemm) with tile shape T.
+template <class S, int OP, class T>
+static void launch_pgemm(BHandle* h, const PGroup& g, int l) {
+  constexpr int RB = (OP == PT_QKV ? S::QKV : (OP == PT_GU ? S::F : S::H)) / 16;
+  static_assert(RB % T::MR == 0, "whole row tiles");
+  static_assert(RB / T::MR % 8 == 0 || RB < 64, "a row tile's workgroups share an XCD and its L2");
+  hipLaunchKernelGGL((bk_pgemm<S, OP, T>), dim3(RB / T::MR, (g.n + T::NG - 1) / T::NG), dim3(T::W * kWave), 0,
+                     h->stream, g, l);
+}
+
+// Tile shapes by the pass's column groups n: the largest that still gives the
+// chip about one workgroup per CU -- a larger tile reads fewer bytes per
+// product, a smaller one starts more workgroups.  (us per layer at n = 2 / 4 /
+// 8 / 16 / 32 / 64; * the range it is used in.)
+//   QKV   2x1   4.4*  4.7*  5.5   7.9  13.6  24.9     O    2x1  4.1*  3.8*  3.9*  5.1   8.2  15.9
+//         2x2   4.6   5.1   5.1*  6.6  10.6  19.0          2x2  4.5   4.4   4.3   4.6*  6.7  11.7
+//         4x2   5.2   5.1   5.2   5.5*  9.5  18.1          4x2  5.0   4.9   5.0   5.1   5.8* 11.1
+//         4x4   6.1   6.7   6.8   7.0   7.8* 13.1          4x4  6.3   6.7   6.8   6.9   7.3   9.6*
+//         8x4   9.2  10.1  10.2  10.5  10.8  12.1*
+//   gate  2x1   6.2*  7.6   9.6  15.3  25.0  46.0     down 1x1  5.1*  5.2*  8.2  14.9  28.1  53.1
+//   / up  2x2   7.3   7.0*  8.9* 11.7* 18.6  30.5          2x1  6.1   6.1   6.3* 11.2  21.3  40.4
+//         2x4   8.0   9.5   9.1  12.0  16.5* 27.6*         2x2  7.5   7.5   7.4   8.0* 15.2  28.1
+//         4x4  11.2  13.2  12.9  12.6  21.6  31.8          4x2  9.6   9.5   9.3   9.7  11.5* 19.7
+//                                                          4x4 10.9  13.5  13.0  13.4  15.1  18.4*
+template <class S>
+static void launch_pgemm_qkv(BHandle* h, const PGroup& g, int l) {
+  if (g.n <= 4) launch_pgemm<S, PT_QKV, PTile<2, 1, 4, 1, 8>>(h, g, l);
+  else if (g.n <= 8) launch_pgemm<S, PT_QKV, PTile<2, 2, 4, 1, 8>>(h, g, l);
+  else if (g.n <= 16) launch_pgemm<S, PT_QKV, PTile<4, 2, 2, 2, 8>>(h, g, l);
+  else if (g.n <= 32) launch_pgemm<S, PT_QKV, PTile<4, 4, 1, 2, 4>>(h, g, l);
+  else launch_pgemm<S, PT_QKV, PTile<8, 4, 1, 2, 4>>(h, g, l);
+}
+template <class S>
+static void launch_pgemm_o(BHandle* h, const PGroup& g, int l) {
+  if (g.n <= 8) launch_pgemm<S, PT_O, PTile<2, 1, 4, 1, 8>>(h, g, l);
+  else if (g.n <= 16) launch_pgemm<S, PT_O, PTile<2, 2, 4, 1, 8>>(h, g, l);
+  else if (g.n <= 32) launch_pgemm<S, PT_O, PTile<4, 2, 2, 2, 8>>(h, g, l);
+  else launch_pgemm<S, PT_O, PTile<4, 4, 1, 2, 8>>(h, g, l);
+}
+template <class S>
+static void launch_pgemm_gu(BHandle* h, const PGroup& g, int l) {
+  if (g.n <= 2) launch_pgemm<S, PT_GU, PTile<2, 1, 4, 1, 8>>(h, g, l);
+  else if (g.n <= 16) launch_pgemm<S, PT_GU, PTile<2, 2, 2, 2, 4>>(h, g, l);
+  else launch_pgemm<S, PT_GU, PTile<2, 4, 1, 2, 4>>(h, g, l);
+}
+template <class S>
+static void launch_pgemm_down(BHandle* h, const PGroup& g, int l) {
+  if (g.n <= 4) launch_pgemm<S, PT_DN, PTile<1, 1, 11, 1, 8>>(h, g, l);
+  else if (g.n <= 8) launch_pgemm<S, PT_DN, PTile<2, 1, 11, 1, 8>>(h, g, l);
+  else if (g.n <= 16) launch_pgemm<S, PT_DN, PTile<2, 2, 3, 2, 8>>(h, g, l);
+  else if (g.n <= 32) launch_pgemm<S, PT_DN, PTile<4, 2, 2, 2, 4>>(h, g, l);
+  else launch_pgemm<S, PT_DN, PTile<4, 4, 1, 2, 4>>(h, g, l);
+}
+
 // One prefill pass: up to PG_MAX column groups of <= 16 consecutive prompt
-// tokens of one sequence (up to 1,024 tokens per pass over the weights): the
-// decode step's kernels with bk_append storing every column's K / V before
-// each layer's attention; the LM head and the token only for the prompt's
-// last pass, on its last group (the one holding the prompt's last token).
+// tokens of one sequence (up to 1,024 tokens per pass over the weights):
+// bk_append stores every column's K / V before each layer's attention; the LM
+// head and the token only for the prompt's last pass, on its last group (the
+// one holding the prompt's last token).
 // pl: the parameters of the pass's last group (the LM head's input when last).
 template <class S>
 static int launch_prefill(BHandle* h, const PGroup& g, const BParams& pl, bool last) {
   const int L = h->L, ng = g.n;
-  const auto rows = [ng](int cg) { return (ng + cg - 1) / cg; };  // GEMM workgroup rows: cg groups each
   const BParams& p = g.p;
   hipLaunchKernelGGL((bk_embed<S, PGroup>), dim3(BMAX, ng), dim3(256), 0, h->stream, g);
   for (int l = 0; l < L; ++l) {
-    if (ng > PT_SMALL_GROUPS)
-      hipLaunchKernelGGL((bk_ptile<S, PT_QKV, PTileQKV>), dim3(S::QKV / 16 / PTileQKV::MP, rows(PTileQKV::NG)),
-                         dim3(GT), 0, h->stream, g, l);
-    else
-      hipLaunchKernelGGL((bk_ptile<S, PT_QKV, PTileQKVs>), dim3(S::QKV / 16 / PTileQKVs::MP, rows(PTileQKVs::NG)),
-                         dim3(GT), 0, h->stream, g, l);
+    launch_pgemm_qkv<S>(h, g, l);
     if (p.kscale) {
       hipLaunchKernelGGL((bk_append<S, true, PGroup>), dim3(BMAX * S::NKV, ng), dim3(2 * kWave), 0, h->stream, g,
                          l);
@@ -145,24 +193,9 @@ static int launch_prefill(BHandle* h, const PGroup& g, const BParams& pl, bool l
                          l);
       hipLaunchKernelGGL((bk_pattn<S, false>), dim3(S::NKV, ng), dim3(PC_AW * kWave), 0, h->stream, g, l);
     }
-    if (ng > PT_SMALL_GROUPS)
-      hipLaunchKernelGGL((bk_ptile<S, PT_O, PTileO>), dim3(S::H / 16 / PTileO::MP, rows(PTileO::NG)), dim3(GT), 0,
-                         h->stream, g, l);
-    else
-      hipLaunchKernelGGL((bk_ptile<S, PT_O, PTileOs>), dim3(S::H / 16 / PTileOs::MP, rows(PTileOs::NG)), dim3(GT), 0,
-                         h->stream, g, l);
-    if (ng > PT_SMALL_GROUPS)
-      hipLaunchKernelGGL((bk_pgu_t<S, PTileGU>), dim3(S::F / 16 / PTileGU::MP, rows(PTileGU::NG)), dim3(GT), 0,
-                         h->stream, g, l);
-    else
-      hipLaunchKernelGGL((bk_pgu_t<S, PTileGUs>), dim3(S::F / 16 / PTileGUs::MP, rows(PTileGUs::NG)), dim3(GT), 0,
-                         h->stream, g, l);
-    if (ng > PT_SMALL_GROUPS)
-      hipLaunchKernelGGL((bk_ptile<S, PT_DN, PTileDN>), dim3(S::H / 16 / PTileDN::MP, rows(PTileDN::NG)), dim3(GT), 0,
-                         h->stream, g, l);
-    else
-      hipLaunchKernelGGL((bk_ptile<S, PT_DN, PTileDNs>), dim3(S::H / 16 / PTileDNs::MP, rows(PTileDNs::NG)), dim3(GT),
-                         0, h->stream, g, l);
+    launch_pgemm_o<S>(h, g, l);
+    launch_pgemm_gu<S>(h, g, l);
+    launch_pgemm_down<S>(h, g, l);
   }
   if (last) {
     if (pl.lmhead8)
@@ -174,12 +207,6 @@ static int launch_prefill(BHandle* h, const PGroup& g, const BParams& pl, bool l
   HIPCHK(hipGetLastError(), -1);
   return 0;
 }
-// QKV, O and down grids of whole XCD rounds: a row tile's column-group
-// workgroups share an XCD and its L2 (gate / up has 44 row tiles: its tiles'
-// groups spread over XCDs)
-static_assert((ShapeBaseline::QKV / 16 / PTileQKV::MP) % 8 == 0 && (ShapeBaseline::H / 16 / PTileO::MP) % 8 == 0 &&
-                  (ShapeBaseline::H / 16 / PTileDN::MP) % 8 == 0,
-              "prefill GEMM grids of whole XCD rounds");
 
 template <class S>
 static bool persistent_fits() {

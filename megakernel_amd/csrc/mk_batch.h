@@ -706,436 +706,189 @@ __global__ __launch_bounds__(GT) void bk_down(G p, int layer) {
 }
 
 // ------------------------------------------------------------ prefill GEMMs
-// A prefill pass has up to 64 column groups (1,024 tokens), so the GEMMs are
-// real matrix products: the decode kernels' one-block workgroups would each
-// re-read their group's activation columns (64 KB for K = 1,024) next to
-// 32 KB of weights, bounded by L2 -> CU traffic.  The prefill kernels tile
-// rows and column groups and stage both operands in LDS.  Per 16 x 16 tile
-// the products are the decode kernels' MFMA tiles (weights as the A operand,
-// the columns' bf16 hi / lo parts as two B operands), accumulated over the
-// whole K by one wave, so no cross-wave reduction is needed.
-
-// Tile shapes: MP row blocks (gate / up: block pairs of 16 gate + 16 up rows)
-// x NG column groups per workgroup, K in chunks of KC tiles; each chunk's
-// weight tiles and column tiles are staged in LDS once (double-buffered, the
-// next chunk's loads in flight during the current chunk's products), so a
-// weight byte is read from L2 once per NG groups and a column byte once per
-// MP blocks.  Wave w owns WB blocks x WGR groups over the whole K; the
-// epilogue runs on its accumulators.
-template <int MP_, int NG_, int KC_, int WB_, int WGR_, int PD_ = 2, int NS_ = 0>
+// A pass has 1 to 64 column groups.  A workgroup of W waves computes MR row
+// blocks (gate / up: block pairs of 16 gate + 16 up rows) x NG groups over the
+// whole K, split over its waves: wave w takes the 1 KiB units w, w + W, ... of
+// every row block and column plane, straight into registers (weights as the A
+// operand, the columns' bf16 hi / lo parts as two B operands of one
+// accumulator), NBUF chunks of CW units in flight.  The waves' sums meet in
+// LDS once, in wave order, and each wave runs the epilogue of its share of the
+// tiles: QKV scales by the group's norm factor, gate / up applies SiLU, O and
+// down add the residual and publish x (the next norm's parts and per-block
+// sums of squares) as publish_x does; the epilogue's inputs are loaded before
+// the product.
+//
+// What bounds it: a short pass the latency of one load round per kernel (23
+// tokens: 4 - 6 us per GEMM, a kernel's fixed cost about 4), a long one the
+// bytes that cross L2 per product.  No barrier and no LDS copy stands between
+// a load and its product, and a wave's loads are all independent, so a
+// workgroup keeps 64 - 256 KiB in flight.  The kernels before this staged both
+// operands in LDS by chunks of K, with a barrier per chunk: every chunk waited
+// for its loads (0.5 - 1.2 us each, 16 to 32 in a row).  us per layer, before
+// -> now:            2 groups     13           32           64
+//   QKV              9.3 -> 4.4   9.6 -> 5.4   10.1 -> 7.8  15.0 -> 12.1
+//   O                8.0 -> 3.8   8.2 -> 4.5    8.7 -> 5.8  11.0 -> 9.6
+//   gate / up       18.7 -> 6.2  23.5 -> 11.4  25.9 -> 16.5 32.5 -> 27.6
+//   down            19.2 -> 5.1  18.3 -> 7.4   19.9 -> 11.5 20.7 -> 18.4
+template <int MR_, int NG_, int CW_, int NBUF_, int W_>
 struct PTile {
-  static constexpr int MP = MP_, NG = NG_, KC = KC_, WB = WB_, WGR = WGR_;
-  static constexpr int PD = PD_;  // K chunks whose loads are in flight (1 or 2 register sets)
-  // NS > 0: no register staging; NS LDS stages filled by direct-to-LDS loads
-  // (pt_pipeline), NS - 1 chunks in flight
-  static constexpr int NS = NS_;
-  static_assert((MP / WB) * (NG / WGR) == GW, "every wave owns whole blocks x groups");
-  static_assert(PD == 1 || PD == 2, "one or two register sets");
-  static_assert(NS == 0 || NS >= 2, "two stages at least");
+  static constexpr int MR = MR_, NG = NG_, CW = CW_, NBUF = NBUF_, W = W_;
 };
-
-// One 16-byte load per lane straight into LDS (global_load_lds_dwordx4):
-// lane l's bytes land at dst + 16 l, dst being the wave's (uniform) address,
-// passed in M0.  It counts on vmcnt like any vector load and writes no
-// register.  Inline assembly, so that the compiler does not add its own
-// conservative wait for every such load in flight before each LDS read: the
-// caller waits for exactly the loads it needs (wait_vmcnt).  M0 is declared
-// clobbered (the compiler warns, M0 being reserved); the GEMM kernels that
-// use this have no other M0 user (no compiler-issued LDS DMA, no indirect
-// register indexing: every register array index is a compile-time constant).
-__device__ __forceinline__ void lds_load16(const void* src, void* dst) {
-  const unsigned m0 = __builtin_amdgcn_readfirstlane(
-      (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)dst);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0), "v"(src) : "memory", "m0");
-}
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N <= 63, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// The K loop of a tiled GEMM over NS LDS stages filled by direct loads:
-// chunk c goes to stage c % NS, issued NS - 1 chunks ahead (issue(c, stage),
-// NI loads per lane).  Before multiplying chunk c a wave waits until its own
-// loads of chunk c have landed (vmcnt: the later chunks' loads may stay in
-// flight); the barrier after it makes every wave's share visible and retires
-// the stage the next issue overwrites (multiplied in the previous iteration,
-// whose LDS reads every wave has consumed before reaching the barrier).  The
-// plain s_barrier: __syncthreads()' fence would wait for every load in
-// flight.
-template <int NS, int NC, int NI, class Issue, class Compute>
-__device__ __forceinline__ void pt_pipeline(const Issue& issue, const Compute& compute) {
-  static_assert(NC >= NS - 1, "the prologue fills NS - 1 stages");
-#pragma unroll
-  for (int c = 0; c < NS - 1; ++c) issue(c, c);
-  for (int c = 0; c < NC; ++c) {
-    if (c + NS - 1 <= NC) wait_vmcnt<(NS - 2) * NI>();
-    else wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (c + NS - 1 < NC) issue(c + NS - 1, (c + NS - 1) % NS);
-    compute(c % NS);
-  }
-  asm volatile("" ::: "memory");
-}
-// (measured per layer, us: gate / up <8,8,2,4,2> 46.5, <8,8,2,2,4> 47.3,
-// <8,8,2,1,8> 50.2, <8,4,2,1,4> 67.4, <4,8,2,1,4> 71.9, <4,4,4,1,2> 61.6;
-// QKV <8,2,2,2,1> 19.5, <8,2,2,1,2> 20.1, <4,4,2,1,2> 22.8, <4,2,4,1,1> 27.5,
-// <4,4,4,1,2> 31.7, <8,8,2,1,8> 33.7; O <4,2,4,1,1> 20.7, <8,1,4,1,1> 20.6,
-// <8,2,4,2,1> 22.1, <4,4,4,1,2> 23.7; down <4,2,4,1,1> 38.5, <8,1,4,1,1> 39.2,
-// <8,2,4,2,1> 41.6, <4,4,4,1,2> 47.7, <2,4,4,1,1> 54.3.  A wave owning more
-// blocks reads fewer LDS bytes per product.)
-// gate / up: direct-to-LDS loads, K chunks of one tile, four stages (three
-// chunks in flight): 44.0 -> 40.3 us against <8,8,2,4,2> with one register
-// set (234 VGPRs)
-using PTileGU = PTile<8, 8, 1, 4, 2, 1, 4>;
-// gate / up of a pass of at most PT_SMALL_GROUPS groups: the 8 x 8 tile
-// leaves too few workgroups (256 tokens: 44), 8 x 2 four times as many
-// (measured, tok/s, 8 x 8 / 8 x 2: 128 tokens 37,869 / 44,851, 256 tokens
-// 74,028 / 87,756, 512 tokens 138,672 / 154,683, 1,024 tokens 220,199 /
-// 207,877)
-using PTileGUs = PTile<8, 2, 2, 2, 1>;
-#ifndef MK_PT_SMALL_GROUPS
-#define MK_PT_SMALL_GROUPS 32
-#endif
-constexpr int PT_SMALL_GROUPS = MK_PT_SMALL_GROUPS;
-// Direct-to-LDS loads (us per layer at 1,024 tokens): QKV three stages of
-// two tiles (four, 96 KB of LDS, leave one workgroup per CU: 18.1 -> 21.1;
-// chunks of four tiles 19.5); O and down 8 x 2 tiles, chunks of four tiles,
-// three stages (144 KB: one workgroup per CU, 256 workgroups): O 20.9 ->
-// 18.9, down 38.4 -> 32.3 (register-staged 4 x 2
-// tiles before; down 4 x 2 with four direct-load stages 38.7, 8 x 2 with
-// chunks of two tiles and three / four / six stages 33.2 / 33.0 / 35.1, 4 x 4
-// 35.8).  Each wave owns 1 block x 2 groups in O and 2 blocks x 1 group in
-// down: with 2 x 1 the epilogue's rows reach memory about twice (17.7 MB
-// written per launch against 8.7 MB of output, WRITE_SIZE), with 1 x 2 once,
-// at the same O time and 0.8 us more for down.
-using PTileQKV = PTile<16, 2, 2, 4, 1, 2, 3>;  // 17.5 -> 16.7 us against 8 x 2 (16 x 2 with chunks of four: 18.9)
-using PTileQKVs = PTile<8, 2, 2, 2, 1, 2, 3>;  // passes of at most PT_SMALL_GROUPS groups
-using PTileO = PTile<8, 2, 4, 1, 2, 2, 3>;  // each wave 1 block x 2 groups (2 x 1 wrote its outputs twice)
-using PTileOs = PTile<4, 2, 2, 1, 1, 2, 4>;  // passes of at most PT_SMALL_GROUPS groups (twice the workgroups)
-using PTileDN = PTile<8, 2, 4, 2, 1, 1, 3>;
-using PTileDNs = PTile<4, 2, 4, 1, 1, 2>;  // passes of at most PT_SMALL_GROUPS groups
-
-template <class S, class T>
-__global__ __launch_bounds__(GT) void bk_pgu_t(PGroup pg, int layer) {
-  constexpr int MP = T::MP, NG = T::NG, KC = T::KC, WB = T::WB, WGR = T::WGR;
-  constexpr int NT = S::KT_H, NC = NT / KC;
-  constexpr int AU = 2 * MP * KC * kWave;  // u32x4 of a chunk's weight tiles
-  constexpr int BU = NG * 2 * KC * kWave;  // ... of its column tiles
-  constexpr int LA = AU / GT, LB = BU / GT;  // per thread
-  static_assert(NT % KC == 0 && AU % GT == 0 && BU % GT == 0, "tile shape");
-  constexpr int NSB = T::NS > 0 ? T::NS : 2;
-  __shared__ u32x4 sa[NSB][2 * MP][KC][kWave];  // [buf][gate blocks | up blocks][tile][lane]
-  __shared__ u32x4 sb[NSB][NG][2][KC][kWave];   // [buf][group][hi / lo][tile][lane]
-  // workgroup i runs on XCD i % 8: tiles (r, c) numbered r * ct + c are dealt
-  // to XCDs in contiguous runs, so a row tile's column tiles share an XCD's L2
-  // (its 22 row tiles are no multiple of 8; with the plain grid order a
-  // launch fetched 83 MB from beyond L2 for 11.5 MB of weights, and the
-  // kernel took 46.3 instead of 44.0 us)
-  const int ct = (int)gridDim.y, nw = (int)gridDim.x * ct, lin = (int)(blockIdx.y * gridDim.x + blockIdx.x);
-  const int jt = nw % 8 == 0 ? (lin % 8) * (nw / 8) + lin / 8 : lin;
-  const int rb0 = (jt / ct) * MP, g0 = (jt % ct) * NG, tid = ltid();
-  const int ngr = pg.n - g0 < NG ? pg.n - g0 : NG;  // groups of this tile
-  const BParams p0 = group_params(pg, g0);
-  const u32x4* wgt[2] = {p0.wg + layer * p0.u_gu, p0.wu + layer * p0.u_gu};
-  u32x4 ra[T::PD][LA], rbv[T::PD][LB];
-  const auto load = [&](int c, u32x4(&xa)[LA], u32x4(&xb)[LB]) {
-#pragma unroll
-    for (int k = 0; k < LA; ++k) {
-      const int i = tid + GT * k, blk = i / (KC * kWave), kt = (i / kWave) % KC, ln = i % kWave;
-      xa[k] = __builtin_nontemporal_load(wgt[blk / MP] + ((long long)(rb0 + blk % MP) * NT + c * KC + kt) * 64 + ln);
-    }
-#pragma unroll
-    for (int k = 0; k < LB; ++k) {
-      const int i = tid + GT * k, gq = i / (2 * KC * kWave), pl = (i / (KC * kWave)) % 2;
-      const int kt = (i / kWave) % KC, ln = i % kWave;
-      xb[k] = u32x4{0u, 0u, 0u, 0u};
-      if (gq < ngr)
-        xb[k] = *reinterpret_cast<const u32x4*>(xg_plane<S>(group_params(pg, g0 + gq), 0, 1, pl) +
-                                                 512 * (c * KC + kt) + 8 * ln);
-    }
-  };
-  const auto store = [&](int buf, const u32x4(&xa)[LA], const u32x4(&xb)[LB]) {
-#pragma unroll
-    for (int k = 0; k < LA; ++k) (&sa[buf][0][0][0])[tid + GT * k] = xa[k];
-#pragma unroll
-    for (int k = 0; k < LB; ++k) (&sb[buf][0][0][0][0])[tid + GT * k] = xb[k];
-  };
-  // direct loads: wave w moves whole 1 KB tiles w, w + 8, ... of a chunk
-  const auto issue = [&](int c, int buf) {
-    const int w = wave_id(), ln = (int)lane_id();
-#pragma unroll
-    for (int k = 0; k < LA; ++k) {
-      const int t = w + GW * k, blk = t / KC, kt = t % KC;
-      lds_load16(wgt[blk / MP] + ((long long)(rb0 + blk % MP) * NT + c * KC + kt) * 64 + ln, &sa[buf][blk][kt][0]);
-    }
-#pragma unroll
-    for (int k = 0; k < LB; ++k) {
-      const int t = w + GW * k, gq = t / (2 * KC), pl = (t / KC) % 2, kt = t % KC;
-      const int gs = gq < ngr ? gq : 0;  // a group past the pass reads group 0 (its columns are never stored)
-      lds_load16(xg_plane<S>(group_params(pg, g0 + gs), 0, 1, pl) + 512 * (c * KC + kt) + 8 * ln,
-                 &sb[buf][gq][pl][kt][0]);
-    }
-  };
-  if constexpr (T::NS == 0) {
-    load(0, ra[0], rbv[0]);
-    store(0, ra[0], rbv[0]);
-    if constexpr (T::PD == 2)
-      if (NC > 1) load(1, ra[T::PD - 1], rbv[T::PD - 1]);
-    __syncthreads();
-  }
-  const int w = wave_id(), pw = (w / (NG / WGR)) * WB, gb = (w % (NG / WGR)) * WGR;
-  const unsigned l = lane_id();
-  f32x4 acc[WB][WGR][2][2];  // [block][group][gate / up][hi / lo part]
-#pragma unroll
-  for (int r = 0; r < WB; ++r)
-#pragma unroll
-    for (int j = 0; j < WGR; ++j)
-#pragma unroll
-      for (int m = 0; m < 2; ++m) acc[r][j][m][0] = acc[r][j][m][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const auto compute = [&](int buf) {
-#pragma unroll
-    for (int kt = 0; kt < KC; ++kt) {
-#pragma unroll
-      for (int r = 0; r < WB; ++r) {
-        const u32x4 ag = sa[buf][pw + r][kt][l], au = sa[buf][MP + pw + r][kt][l];
-#pragma unroll
-        for (int j = 0; j < WGR; ++j) {
-          const u32x4 bh = sb[buf][gb + j][0][kt][l], bl = sb[buf][gb + j][1][kt][l];
-          acc[r][j][0][0] = mfma(ag, bh, acc[r][j][0][0]);
-          acc[r][j][0][1] = mfma(ag, bl, acc[r][j][0][1]);
-          acc[r][j][1][0] = mfma(au, bh, acc[r][j][1][0]);
-          acc[r][j][1][1] = mfma(au, bl, acc[r][j][1][1]);
-        }
-      }
-    }
-  };
-  if constexpr (T::NS > 0) {
-    pt_pipeline<T::NS, NC, LA + LB>(issue, compute);
-  } else if constexpr (T::PD == 1) {
-    for (int c = 0; c < NC; ++c) {
-      if (c + 1 < NC) load(c + 1, ra[0], rbv[0]);
-      compute(c & 1);
-      if (c + 1 < NC) store((c + 1) & 1, ra[0], rbv[0]);
-      __syncthreads();
-    }
-  } else {
-    // chunk k sits in register set k & 1, then in LDS buffer k & 1: while a
-    // chunk is multiplied, the next one waits in registers and the one after
-    // it is loading
-    for (int c = 0; c < NC; c += 2) {
-      if (c + 2 < NC) load(c + 2, ra[0], rbv[0]);
-      compute(0);
-      if (c + 1 < NC) store(1, ra[T::PD - 1], rbv[T::PD - 1]);
-      __syncthreads();
-      if (c + 1 >= NC) break;
-      if (c + 3 < NC) load(c + 3, ra[T::PD - 1], rbv[T::PD - 1]);
-      compute(1);
-      if (c + 2 < NC) store(0, ra[0], rbv[0]);
-      __syncthreads();
-    }
-  }
-  // epilogue: lane (kg, n) holds rows 4 kg .. 4 kg + 3 of column n
-  const int n = (int)(l & 15u), kg = (int)(l >> 4);
-#pragma unroll
-  for (int j = 0; j < WGR; ++j) {
-    if (gb + j >= ngr) break;
-    const BParams p = group_params(pg, g0 + gb + j);
-    constexpr int NB = S::H / 16, PER = NB / 4;
-    const float* q = ssq_slot<S>(p, 0, 1) + n;
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) ss += q[(kg * PER + i) * BMAX];
-    ss = sum_xor32(sum_xor16(ss));
-    const float rs = rsqrtf(ss / (float)S::H + kRmsEps);
-    if (n < p.B) {
-#pragma unroll
-      for (int r = 0; r < WB; ++r) {
-        uint16_t h[4], o[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float g = (acc[r][j][0][0][i] + acc[r][j][0][1][i]) * rs;
-          const float u = (acc[r][j][1][0][i] + acc[r][j][1][1][i]) * rs;
-          split2(g / (1.0f + __expf(-g)) * u, h[i], o[i]);  // SiLU(g) * u (reference utils.cuh:59-61)
-        }
-        uint16_t* a = act_slot<S>(p, 0) + unit_at(n, (rb0 + pw + r) * 16 + 4 * kg);
-        st4(a, h);
-        st4(a + BMAX * S::F, o);
-      }
-    }
-  }
-}
-
-// QKV, O and down as LDS-tiled GEMMs, as bk_pgu_t with one weight matrix.
-// Epilogues: QKV scales by the
-// group's norm factor; O and down add the residual and publish x (the next
-// norm's bf16 parts and per-block sums of squares) as publish_x does.
-enum PtOp : int { PT_QKV = 0, PT_O = 1, PT_DN = 2 };
+enum PtOp : int { PT_QKV = 0, PT_O = 1, PT_DN = 2, PT_GU = 3 };
 template <class S, int OP, class T>
-__global__ __launch_bounds__(GT) void bk_ptile(PGroup pg, int layer) {
-  constexpr int MP = T::MP, NG = T::NG, KC = T::KC, WB = T::WB, WGR = T::WGR;
-  constexpr int K = OP == PT_QKV ? S::H : (OP == PT_O ? S::QD : S::F);
-  constexpr int NT = K / 32, NC = NT / KC;
-  constexpr int AU = MP * KC * kWave, BU = NG * 2 * KC * kWave;
-  constexpr int LA = AU / GT, LB = BU / GT;
-  static_assert(NT % KC == 0 && AU % GT == 0 && BU % GT == 0, "tile shape");
-  constexpr int NSB = T::NS > 0 ? T::NS : 2;
-  __shared__ u32x4 sa[NSB][MP][KC][kWave];
-  __shared__ u32x4 sb[NSB][NG][2][KC][kWave];
-  const int rb0 = blockIdx.x * MP, g0 = blockIdx.y * NG, tid = ltid();
-  const int ngr = pg.n - g0 < NG ? pg.n - g0 : NG;
+__global__ __launch_bounds__(T::W * kWave) void bk_pgemm(PGroup pg, int layer) {
+  constexpr int MR = T::MR, NGW = T::NG, W = T::W;
+  constexpr bool GU = OP == PT_GU;
+  constexpr int NB = GU ? 2 : 1;  // blocks per row tile
+  constexpr int K = OP == PT_O ? S::QD : (OP == PT_DN ? S::F : S::H);
+  constexpr int NT = K / 32, TW = NT / W, CW = T::CW < TW ? T::CW : TW;
+  constexpr int NCH = (TW + CW - 1) / CW, NBUF = T::NBUF < NCH ? T::NBUF : NCH;
+  static_assert(NT % W == 0, "whole units per wave");
+  constexpr int TL = MR * NGW, TPW = (TL + W - 1) / W;  // row tile x group pairs, per wave
+  __shared__ f32x4 red[W][TL][NB][kWave];
+  const int rb0 = blockIdx.x * MR, g0 = blockIdx.y * NGW;
+  const int ngr = pg.n - g0 < NGW ? pg.n - g0 : NGW;
+  const int w = wave_id(), l = (int)lane_id();
+  const int n = l & 15, kg = l >> 4;
   const BParams p0 = group_params(pg, g0);
-  const u32x4* wm = OP == PT_QKV ? p0.wqkv + layer * p0.u_qkv
-                                 : (OP == PT_O ? p0.wo + layer * p0.u_o : p0.wd + layer * p0.u_dn);
-  // column planes of group q: hi at plane(q, 0), lo at plane(q, 1), [BMAX][K]
-  const auto plane = [&](const BParams& q, int pl) -> const uint16_t* {
-    if constexpr (OP == PT_QKV) return xg_plane<S>(q, 0, 0, pl);
-    if constexpr (OP == PT_O) return att_slot<S>(q, 0) + (long long)pl * BMAX * S::QD;
-    return act_slot<S>(q, 0) + (long long)pl * BMAX * S::F;
-  };
-  u32x4 ra[T::PD][LA], rbv[T::PD][LB];
-  const auto load = [&](int c, u32x4(&xa)[LA], u32x4(&xb)[LB]) {
+  const long long gs = pg.gstride;
+  const u32x4* wm[NB];
+  if constexpr (GU) wm[0] = p0.wg + layer * p0.u_gu, wm[1] = p0.wu + layer * p0.u_gu;
+  else wm[0] = OP == PT_QKV ? p0.wqkv + layer * p0.u_qkv : (OP == PT_O ? p0.wo + layer * p0.u_o : p0.wd + layer * p0.u_dn);
+  const uint16_t* pl = OP == PT_QKV ? xg_plane<S>(p0, 0, 0, 0)
+                                    : (GU ? xg_plane<S>(p0, 0, 1, 0) : (OP == PT_O ? att_slot<S>(p0, 0) : act_slot<S>(p0, 0)));
+  // the epilogue's inputs first: the norm's block sums, or the residual rows
+  constexpr bool NORM = OP == PT_QKV || GU;
+  constexpr int NSB = S::H / 16, PER = NSB / 4;
+  constexpr int CI = OP == PT_O ? 0 : 1, CO = 1 - CI;
+  float sv[NORM ? TPW : 1][PER];
+  f32x4 xr[TPW];
+  u32x2 gw[TPW];
+  const uint16_t* gain = OP == PT_O ? p0.norms + (long long)layer * S::NORM_STRIDE + S::NORM_FFN
+                                    : (layer + 1 < p0.L ? p0.norms + (long long)(layer + 1) * S::NORM_STRIDE + S::NORM_ATTN
+                                                        : p0.final_norm);
 #pragma unroll
-    for (int k = 0; k < LA; ++k) {
-      const int i = tid + GT * k, blk = i / (KC * kWave), kt = (i / kWave) % KC, ln = i % kWave;
-      xa[k] = __builtin_nontemporal_load(wm + ((long long)(rb0 + blk) * NT + c * KC + kt) * 64 + ln);
+  for (int i = 0; i < TPW; ++i) {
+    const int t = w + W * i, j = t / MR < ngr ? t / MR : 0;
+    if constexpr (NORM) {
+      const float* q = advance(ssq_slot<S>(p0, 0, GU ? 1 : 0), j * gs) + n;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) sv[i][e] = q[(kg * PER + e) * BMAX];
+    } else {
+      const int row = (rb0 + t % MR) * 16 + 4 * kg;
+      xr[i] = *reinterpret_cast<const f32x4*>(advance(x_slot<S>(p0, 0, CI), j * gs) + x_at(n, row));
+      gw[i] = *reinterpret_cast<const u32x2*>(gain + row);
     }
-#pragma unroll
-    for (int k = 0; k < LB; ++k) {
-      const int i = tid + GT * k, gq = i / (2 * KC * kWave), pl = (i / (KC * kWave)) % 2;
-      const int kt = (i / kWave) % KC, ln = i % kWave;
-      xb[k] = u32x4{0u, 0u, 0u, 0u};
-      if (gq < ngr)
-        xb[k] = *reinterpret_cast<const u32x4*>(plane(group_params(pg, g0 + gq), pl) + 512 * (c * KC + kt) + 8 * ln);
-    }
-  };
-  const auto store = [&](int buf, const u32x4(&xa)[LA], const u32x4(&xb)[LB]) {
-#pragma unroll
-    for (int k = 0; k < LA; ++k) (&sa[buf][0][0][0])[tid + GT * k] = xa[k];
-#pragma unroll
-    for (int k = 0; k < LB; ++k) (&sb[buf][0][0][0][0])[tid + GT * k] = xb[k];
-  };
-  // direct loads: wave w moves whole 1 KB tiles w, w + 8, ... of a chunk
-  const auto issue = [&](int c, int buf) {
-    const int w = wave_id(), ln = (int)lane_id();
-#pragma unroll
-    for (int k = 0; k < LA; ++k) {
-      const int t = w + GW * k, blk = t / KC, kt = t % KC;
-      lds_load16(wm + ((long long)(rb0 + blk) * NT + c * KC + kt) * 64 + ln, &sa[buf][blk][kt][0]);
-    }
-#pragma unroll
-    for (int k = 0; k < LB; ++k) {
-      const int t = w + GW * k, gq = t / (2 * KC), pl = (t / KC) % 2, kt = t % KC;
-      const int gs = gq < ngr ? gq : 0;  // a group past the pass reads group 0 (its columns are never stored)
-      lds_load16(plane(group_params(pg, g0 + gs), pl) + 512 * (c * KC + kt) + 8 * ln, &sb[buf][gq][pl][kt][0]);
-    }
-  };
-  if constexpr (T::NS == 0) {
-    load(0, ra[0], rbv[0]);
-    store(0, ra[0], rbv[0]);
-    if constexpr (T::PD == 2)
-      if (NC > 1) load(1, ra[T::PD - 1], rbv[T::PD - 1]);
-    __syncthreads();
   }
-  const int w = wave_id(), pw = (w / (NG / WGR)) * WB, gb = (w % (NG / WGR)) * WGR;
-  const unsigned l = lane_id();
-  f32x4 acc[WB][WGR][2];  // [block][group][hi / lo part]
+  f32x4 acc[MR][NB][NGW];
 #pragma unroll
-  for (int r = 0; r < WB; ++r)
+  for (int r = 0; r < MR; ++r)
 #pragma unroll
-    for (int j = 0; j < WGR; ++j) acc[r][j][0] = acc[r][j][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const auto compute = [&](int buf) {
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int kt = 0; kt < KC; ++kt) {
+      for (int j = 0; j < NGW; ++j) acc[r][b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 a[NBUF][CW][MR][NB], bh[NBUF][CW][NGW], bl[NBUF][CW][NGW];
+  const auto issue = [&](int c, int q) __attribute__((always_inline)) {
 #pragma unroll
-      for (int r = 0; r < WB; ++r) {
-        const u32x4 a = sa[buf][pw + r][kt][l];
+    for (int u = 0; u < CW; ++u) {
+      if (c * CW + u >= TW) break;
+      const int kt = w + W * (c * CW + u);
 #pragma unroll
-        for (int j = 0; j < WGR; ++j) {
-          acc[r][j][0] = mfma(a, sb[buf][gb + j][0][kt][l], acc[r][j][0]);
-          acc[r][j][1] = mfma(a, sb[buf][gb + j][1][kt][l], acc[r][j][1]);
-        }
+      for (int r = 0; r < MR; ++r)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) a[q][u][r][b] = *(wm[b] + ((long long)(rb0 + r) * NT + kt) * 64 + l);
+#pragma unroll
+      for (int j = 0; j < NGW; ++j) {
+        const uint16_t* s = pl + (j < ngr ? j : 0) * (gs / 2) + 512 * kt + 8 * l;
+        bh[q][u][j] = *reinterpret_cast<const u32x4*>(s);
+        bl[q][u][j] = *reinterpret_cast<const u32x4*>(s + BMAX * K);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
   };
-  if constexpr (T::NS > 0) {
-    pt_pipeline<T::NS, NC, LA + LB>(issue, compute);
-  } else if constexpr (T::PD == 1) {
-    for (int c = 0; c < NC; ++c) {
-      if (c + 1 < NC) load(c + 1, ra[0], rbv[0]);
-      compute(c & 1);
-      if (c + 1 < NC) store((c + 1) & 1, ra[0], rbv[0]);
-      __syncthreads();
-    }
-  } else {
-    // chunk k sits in register set k & 1, then in LDS buffer k & 1: while a
-    // chunk is multiplied, the next one waits in registers and the one after
-    // it is loading
-    for (int c = 0; c < NC; c += 2) {
-      if (c + 2 < NC) load(c + 2, ra[0], rbv[0]);
-      compute(0);
-      if (c + 1 < NC) store(1, ra[T::PD - 1], rbv[T::PD - 1]);
-      __syncthreads();
-      if (c + 1 >= NC) break;
-      if (c + 3 < NC) load(c + 3, ra[T::PD - 1], rbv[T::PD - 1]);
-      compute(1);
-      if (c + 2 < NC) store(0, ra[0], rbv[0]);
-      __syncthreads();
-    }
-  }
-  // epilogue: lane (kg, n) holds rows 4 kg .. 4 kg + 3 of column n
-  const int n = (int)(l & 15u), kg = (int)(l >> 4);
 #pragma unroll
-  for (int j = 0; j < WGR; ++j) {
-    if (gb + j >= ngr) break;
-    const BParams p = group_params(pg, g0 + gb + j);
+  for (int c = 0; c < NBUF; ++c) issue(c, c);
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int q = c % NBUF;
+#pragma unroll
+    for (int u = 0; u < CW; ++u) {
+      if (c * CW + u >= TW) break;
+#pragma unroll
+      for (int r = 0; r < MR; ++r)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int j = 0; j < NGW; ++j) acc[r][b][j] = mfma(a[q][u][r][b], bh[q][u][j], acc[r][b][j]);
+#pragma unroll
+      for (int r = 0; r < MR; ++r)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int j = 0; j < NGW; ++j) acc[r][b][j] = mfma(a[q][u][r][b], bl[q][u][j], acc[r][b][j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (c + NBUF < NCH) issue(c + NBUF, q);
+  }
+#pragma unroll
+  for (int r = 0; r < MR; ++r)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int j = 0; j < NGW; ++j) red[w][j * MR + r][b][l] = acc[r][b][j];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < TPW; ++i) {
+    const int t = w + W * i, j = t / MR, rb = rb0 + t % MR;
+    if (t >= TL || j >= ngr) break;
+    f32x4 v[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      v[b] = red[0][t][b][l];
+#pragma unroll
+      for (int k = 1; k < W; ++k) v[b] += red[k][t][b][l];
+    }
+    const BParams p = group_params(pg, g0 + j);
     const bool on = n < p.B;
-    if constexpr (OP == PT_QKV) {
-      constexpr int NB = S::H / 16, PER = NB / 4;
-      const float* q = ssq_slot<S>(p, 0, 0) + n;
+    const int row = rb * 16 + 4 * kg;
+    if constexpr (NORM) {
       float ss = 0.f;
 #pragma unroll
-      for (int i = 0; i < PER; ++i) ss += q[(kg * PER + i) * BMAX];
+      for (int e = 0; e < PER; ++e) ss += sv[i][e];
       ss = sum_xor32(sum_xor16(ss));
       const float rs = rsqrtf(ss / (float)S::H + kRmsEps);
-      if (on) {
+      if constexpr (GU) {
+        uint16_t h[4], o[4];
 #pragma unroll
-        for (int r = 0; r < WB; ++r)
-          *reinterpret_cast<f32x4*>(qkv_slot<S>(p, 0) + (long long)n * S::QKV + (rb0 + pw + r) * 16 + 4 * kg) =
-              (acc[r][j][0] + acc[r][j][1]) * rs;
+        for (int e = 0; e < 4; ++e) {
+          const float g = v[0][e] * rs, u = v[NB - 1][e] * rs;
+          split2(g / (1.0f + __expf(-g)) * u, h[e], o[e]);  // SiLU(g) * u (reference utils.cuh:59-61)
+        }
+        if (on) {
+          uint16_t* q = act_slot<S>(p, 0) + unit_at(n, row);
+          st4(q, h);
+          st4(q + BMAX * S::F, o);
+        }
+      } else {
+        if (on) *reinterpret_cast<f32x4*>(qkv_slot<S>(p, 0) + (long long)n * S::QKV + row) = v[0] * rs;
       }
     } else {
-      // O: residual stream copy 0 in, copy 1 + the FFN norm's parts out;
-      // down: copy 1 in, copy 0 + the next layer's (or the final) norm out
-      constexpr int CI = OP == PT_O ? 0 : 1, CO = 1 - CI;
-      const uint16_t* gain = OP == PT_O ? p.norms + (long long)layer * S::NORM_STRIDE + S::NORM_FFN
-                                        : (layer + 1 < p.L ? p.norms + (long long)(layer + 1) * S::NORM_STRIDE +
-                                                                 S::NORM_ATTN
-                                                           : p.final_norm);
+      f32x4 xn = xr[i] + v[0];
+      uint16_t h[4], o[4];
+      float sq = 0.f;
 #pragma unroll
-      for (int r = 0; r < WB; ++r) {
-        const int rb = rb0 + pw + r;
-        float sq = 0.f;
-        const int row = rb * 16 + 4 * kg;
-        f32x4 xn = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (on) {
-          xn = *reinterpret_cast<const f32x4*>(x_slot<S>(p, 0, CI) + x_at(n, row));
-          const u32x2 gw = *reinterpret_cast<const u32x2*>(gain + row);
-          uint16_t h[4], o[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            xn[i] += acc[r][j][0][i] + acc[r][j][1][i];
-            split2(xn[i] * bf16_to_f32((uint16_t)(gw[i / 2] >> (16 * (i & 1)))), h[i], o[i]);
-          }
-          *reinterpret_cast<f32x4*>(x_slot<S>(p, 0, CO) + x_at(n, row)) = xn;
-          st4(xg_plane<S>(p, 0, CO, 0) + unit_at(n, row), h);
-          st4(xg_plane<S>(p, 0, CO, 1) + unit_at(n, row), o);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sq += xn[i] * xn[i];
-        sq = sum_xor32(sum_xor16(sq));
-        if (kg == 0) ssq_slot<S>(p, 0, CO)[(long long)rb * BMAX + n] = sq;
+      for (int e = 0; e < 4; ++e) {
+        if (!on) xn[e] = 0.f;
+        split2(xn[e] * bf16_to_f32((uint16_t)(gw[i][e / 2] >> (16 * (e & 1)))), h[e], o[e]);
+        sq += xn[e] * xn[e];
       }
+      if (on) {
+        *reinterpret_cast<f32x4*>(x_slot<S>(p, 0, CO) + x_at(n, row)) = xn;
+        st4(xg_plane<S>(p, 0, CO, 0) + unit_at(n, row), h);
+        st4(xg_plane<S>(p, 0, CO, 1) + unit_at(n, row), o);
+      }
+      sq = sum_xor32(sum_xor16(sq));
+      if (kg == 0) ssq_slot<S>(p, 0, CO)[(long long)rb * BMAX + n] = sq;
     }
   }
 }

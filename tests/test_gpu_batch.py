@@ -307,10 +307,8 @@ def test_batch_prefill_baseline_2l_two_passes():
 
 def test_batch_prefill_baseline_2l_odd_large_pass():
     """A pass of 33 column groups (520 tokens after a 37-position prefix): the
-    large-pass GEMM tiles (more than 32 groups) with column tiles that are
-    only partly filled (2-group tiles of QKV / O / down and 8-group tiles of
-    gate / up each end on one group, the last group half full), so the
-    direct-to-LDS K loops load a stand-in group for the missing ones."""
+    large-pass GEMM tiles (more than 32 groups), whose last column tile holds
+    one group, half full, and loads a stand-in for the missing ones."""
     shape = BASELINE.with_(n_layers=2, vocab=4096)
     dw, eng, _, _ = _prefill_case(shape, 46, prefix=37, prompt_len=520, other_len=3, max_seq=600)
     eng.close()
@@ -618,6 +616,40 @@ def test_batch_full_model_bench_workload_graph(step):
             rel = [float(np.linalg.norm(gf[l] - wf[l]) / np.linalg.norm(wf[l])) for l in range(s.n_layers)]
             _print(f"  seq {b}: appended KV worst layer rel-L2 {max(rel):.2e}")
             assert max(rel) <= 1e-2, f"seq {b}: appended KV rel-L2 {max(rel):.3e}"
+    finally:
+        eng.close()
+        dw.free()
+
+
+@pytest.mark.parametrize("which", ["tiny", "baseline_2l"])
+def test_prefill_tile_shapes_agree(which):
+    """Every GEMM tile shape of a prefill pass (chosen by its column groups:
+    edges of each range, partly filled last groups and tiles) against the same
+    prompt consumed 16 tokens at a time, the shape the oracle tests pin.  The
+    sums of a column are the same numbers in another order: fp32 logits within
+    1e-3 of their RMS, which also covers a bf16 cache row rounding the other way."""
+    shape = {"tiny": TINY, "baseline_2l": BASELINE.with_(n_layers=2, vocab=4096)}[which]
+    dw = DeviceWeights(shape, 5, gain_std=0.1)
+    eng = BatchEngine(dw, 1, 1152, shape)
+    try:
+        prompt = [(37 * i * i + 11 * i + 3) % shape.vocab for i in range(1024)]
+        want, at = {}, 0
+        sizes = [16, 31, 33, 64, 65, 127, 129, 256, 257, 511, 513, 1000, 1024]
+        eng.set_pos(0, 0)
+        while at < 1024:  # the reference logits after every prefix in sizes
+            stop = min([n for n in sizes if n > at] + [at + 16])
+            stop = min(stop, at + 16)
+            tok, logits = eng.prefill(0, prompt[at:stop], with_logits=True)
+            want[stop] = (tok, logits)
+            at = stop
+        for n in sizes:
+            eng.set_pos(0, 0)
+            tok, logits = eng.prefill(0, prompt[:n], with_logits=True)
+            rms = float(np.sqrt(np.mean(want[n][1].astype(np.float64) ** 2)))
+            err = float(np.abs(logits - want[n][1]).max()) / rms
+            assert err < 1e-3, f"{n} tokens: logits off by {err:.2e} of their RMS"
+            top = np.sort(want[n][1])[-2:]
+            assert tok == want[n][0] or top[1] - top[0] < 2e-3 * rms
     finally:
         eng.close()
         dw.free()
