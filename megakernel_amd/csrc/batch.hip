@@ -143,8 +143,7 @@ static void launch_pgemm(BHandle* h, const PGroup& g, int l) {
 //                                                          4x4 10.9  13.5  13.0  13.4  15.1  18.4*
 template <class S>
 static void launch_pgemm_qkv(BHandle* h, const PGroup& g, int l) {
-  if (g.n <= 4) launch_pgemm<S, PT_QKV, PTile<2, 1, 4, 1, 8>>(h, g, l);
-  else if (g.n <= 8) launch_pgemm<S, PT_QKV, PTile<2, 2, 4, 1, 8>>(h, g, l);
+  if (g.n <= 8) launch_pgemm<S, PT_QKV, PTile<4, 1, 4, 1, 8>>(h, g, l);
   else if (g.n <= 16) launch_pgemm<S, PT_QKV, PTile<4, 2, 2, 2, 8>>(h, g, l);
   else if (g.n <= 32) launch_pgemm<S, PT_QKV, PTile<4, 4, 1, 2, 4>>(h, g, l);
   else launch_pgemm<S, PT_QKV, PTile<8, 4, 1, 2, 4>>(h, g, l);
@@ -173,8 +172,8 @@ static void launch_pgemm_down(BHandle* h, const PGroup& g, int l) {
 
 // One prefill pass: up to PG_MAX column groups of <= 16 consecutive prompt
 // tokens of one sequence (up to 1,024 tokens per pass over the weights):
-// bk_append stores every column's K / V before each layer's attention; the LM
-// head and the token only for the prompt's last pass, on its last group (the
+// the QKV kernel stores every column's K / V before the layer's attention; the
+// LM head and the token only for the prompt's last pass, on its last group (the
 // one holding the prompt's last token).
 // pl: the parameters of the pass's last group (the LM head's input when last).
 template <class S>
@@ -184,15 +183,10 @@ static int launch_prefill(BHandle* h, const PGroup& g, const BParams& pl, bool l
   hipLaunchKernelGGL((bk_embed<S, PGroup>), dim3(BMAX, ng), dim3(256), 0, h->stream, g);
   for (int l = 0; l < L; ++l) {
     launch_pgemm_qkv<S>(h, g, l);
-    if (p.kscale) {
-      hipLaunchKernelGGL((bk_append<S, true, PGroup>), dim3(BMAX * S::NKV, ng), dim3(2 * kWave), 0, h->stream, g,
-                         l);
+    if (p.kscale)
       hipLaunchKernelGGL((bk_pattn<S, true>), dim3(S::NKV, ng), dim3(PC_AW * kWave), 0, h->stream, g, l);
-    } else {
-      hipLaunchKernelGGL((bk_append<S, false, PGroup>), dim3(BMAX * S::NKV, ng), dim3(2 * kWave), 0, h->stream, g,
-                         l);
+    else
       hipLaunchKernelGGL((bk_pattn<S, false>), dim3(S::NKV, ng), dim3(PC_AW * kWave), 0, h->stream, g, l);
-    }
     launch_pgemm_o<S>(h, g, l);
     launch_pgemm_gu<S>(h, g, l);
     launch_pgemm_down<S>(h, g, l);

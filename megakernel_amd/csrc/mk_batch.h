@@ -114,7 +114,7 @@ struct BParams {
   unsigned long long timeout_ticks;  // bk_step: wall-clock ticks a hand-off wait may take
   int B, L, V, nsplit_max, max_steps;
   int prefill;              // 1: the columns are consecutive prompt tokens of one sequence whose
-                            //    K / V bk_append has already stored (kv_seq = 0, shared cache)
+                            //    K / V the QKV kernel has already stored (kv_seq = 0, shared cache)
 };
 
 // Up to PG_MAX column groups that share one pass over the weights: a prefill
@@ -713,8 +713,8 @@ __global__ __launch_bounds__(GT) void bk_down(G p, int layer) {
 // operand, the columns' bf16 hi / lo parts as two B operands of one
 // accumulator), NBUF chunks of CW units in flight.  The waves' sums meet in
 // LDS once, in wave order, and each wave runs the epilogue of its share of the
-// tiles: QKV scales by the group's norm factor, gate / up applies SiLU, O and
-// down add the residual and publish x (the next norm's parts and per-block
+// tiles: QKV scales by the group's norm factor and finishes whole heads
+// (qkv_head), gate / up applies SiLU, O and down add the residual and publish x (the next norm's parts and per-block
 // sums of squares) as publish_x does; the epilogue's inputs are loaded before
 // the product.
 //
@@ -735,6 +735,108 @@ struct PTile {
   static constexpr int MR = MR_, NG = NG_, CW = CW_, NBUF = NBUF_, W = W_;
 };
 enum PtOp : int { PT_QKV = 0, PT_O = 1, PT_DN = 2, PT_GU = 3 };
+// One head (D = 64 rows, four row blocks) of the fused QKV product for the 16
+// columns of a group, in one wave: lane (kg, n) holds rows 16 r + 4 kg + i of
+// column n in v[r][i], so a head's sum of squares takes two cross-lane steps
+// and a RoPE pair (d, d + 32) sits in one lane.  q: RMSNorm and RoPE (reference
+// rmsnorm.cuh:57-84, attention.cuh:22-44), fp32 for the attention; k the same,
+// then into the cache like v (reference kv_cache.cuh:58-78) -- before the
+// attention kernel, so that a column sees the columns before it.  (A kernel of
+// its own for k and v took 4.0 - 5.6 us per layer, and every attention
+// workgroup normalised and rotated its queries again: 1,024 tokens 3,277 us,
+// and 2,905 with both here.)
+struct HeadIn {
+  f32x4 cs[2], sn[2];  // RoPE cos / sin of dims 16 r + 4 kg + i, r = 0, 1
+  u32x2 gain[4];       // QK-norm gains of the lane's rows
+};
+template <class S>
+__device__ __forceinline__ void head_load(const BParams& p, int layer, int head, int n, int kg, HeadIn& in) {
+  static_assert(S::D == 64, "heads of four row blocks");
+  const uint16_t* g = p.norms + (long long)layer * S::NORM_STRIDE + (head < S::NQ ? S::NORM_Q : S::NORM_K);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) in.gain[r] = *reinterpret_cast<const u32x2*>(g + 16 * r + 4 * kg);
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    in.cs[r] = *reinterpret_cast<const f32x4*>(p.rope + (n * 2 + 0) * (S::D / 2) + 16 * r + 4 * kg);
+    in.sn[r] = *reinterpret_cast<const f32x4*>(p.rope + (n * 2 + 1) * (S::D / 2) + 16 * r + 4 * kg);
+  }
+}
+template <class S>
+__device__ __forceinline__ void qkv_head(const BParams& p, int layer, int head, int n, int kg, bool on, const HeadIn& in,
+                                         f32x4 (&v)[4]) {
+  constexpr int D = S::D;
+  if (head < S::NQ + S::NKV) {
+    float ss = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ss += v[r][i] * v[r][i];
+    ss = sum_xor32(sum_xor16(ss));
+    const float rn = rsqrtf(ss / (float)D + kRmsEps);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[r][i] = v[r][i] * rn * bf16_to_f32((uint16_t)(in.gain[r][i / 2] >> (16 * (i & 1))));
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float a = v[r][i], b = v[r + 2][i];
+        v[r][i] = a * in.cs[r][i] - b * in.sn[r][i];
+        v[r + 2][i] = b * in.cs[r][i] + a * in.sn[r][i];
+      }
+  }
+  if (head < S::NQ) {
+    if (!on) return;
+    float* q = qkv_slot<S>(p, 0) + (long long)n * S::QKV + head * D + 4 * kg;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) *reinterpret_cast<f32x4*>(q + 16 * r) = v[r];
+    return;
+  }
+  const bool isk = head < S::NQ + S::NKV;
+  const int g = head - S::NQ - (isk ? 0 : S::NKV);
+  const int pos = on ? p.pos[n] : 0;
+  const long long base = ((long long)layer * S::NKV + g) * (long long)p.s_pad;
+  const long long at = isk ? (base + pos) * D + 4 * kg : (base + pos / 32 * 32) * D + (long long)(4 * kg) * 32 + pos % 32;
+  if (p.kscale) {  // FP8 row: codes and the power-of-two scale from the row's maximum
+    float m = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m = fmaxf(m, fabsf(v[r][i]));
+    const int e = e4m3_row_exp(max_xor32(max_xor16(m)));
+    if (!on) return;
+    uint8_t* c = reinterpret_cast<uint8_t*>(isk ? p.kv : p.kvt) + at;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      uint8_t b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = (uint8_t)e4m3_encode(ldexpf(v[r][i], -e));
+      if (isk) {
+        *reinterpret_cast<uint32_t*>(c + 16 * r) = b[0] | (unsigned)b[1] << 8 | (unsigned)b[2] << 16 | (unsigned)b[3] << 24;
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[(16 * r + i) * 32] = b[i];
+      }
+    }
+    if (kg == 0) (isk ? p.kscale : p.vscale)[base + pos] = ldexpf(1.f, e);
+  } else if (on) {
+    uint16_t* c = (isk ? p.kv : p.kvt) + at;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      uint16_t b[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = f32_to_bf16(v[r][i]);
+      if (isk) {
+        st4(c + 16 * r, b);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[(16 * r + i) * 32] = b[i];
+      }
+    }
+  }
+}
+
 template <class S, int OP, class T>
 __global__ __launch_bounds__(T::W * kWave) void bk_pgemm(PGroup pg, int layer) {
   constexpr int MR = T::MR, NGW = T::NG, W = T::W;
@@ -744,8 +846,11 @@ __global__ __launch_bounds__(T::W * kWave) void bk_pgemm(PGroup pg, int layer) {
   constexpr int NT = K / 32, TW = NT / W, CW = T::CW < TW ? T::CW : TW;
   constexpr int NCH = (TW + CW - 1) / CW, NBUF = T::NBUF < NCH ? T::NBUF : NCH;
   static_assert(NT % W == 0, "whole units per wave");
-  constexpr int TL = MR * NGW, TPW = (TL + W - 1) / W;  // row tile x group pairs, per wave
-  __shared__ f32x4 red[W][TL][NB][kWave];
+  // epilogue units of a wave: one row tile, or for QKV one head, of a group
+  constexpr int RU = OP == PT_QKV ? 4 : 1, MU = MR / RU;
+  static_assert(MR % RU == 0, "whole heads");
+  constexpr int TL = MU * NGW, TPW = (TL + W - 1) / W;
+  __shared__ f32x4 red[W][MR * NGW][NB][kWave];
   const int rb0 = blockIdx.x * MR, g0 = blockIdx.y * NGW;
   const int ngr = pg.n - g0 < NGW ? pg.n - g0 : NGW;
   const int w = wave_id(), l = (int)lane_id();
@@ -764,18 +869,20 @@ __global__ __launch_bounds__(T::W * kWave) void bk_pgemm(PGroup pg, int layer) {
   float sv[NORM ? TPW : 1][PER];
   f32x4 xr[TPW];
   u32x2 gw[TPW];
+  HeadIn hin[OP == PT_QKV ? TPW : 1];
   const uint16_t* gain = OP == PT_O ? p0.norms + (long long)layer * S::NORM_STRIDE + S::NORM_FFN
                                     : (layer + 1 < p0.L ? p0.norms + (long long)(layer + 1) * S::NORM_STRIDE + S::NORM_ATTN
                                                         : p0.final_norm);
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
-    const int t = w + W * i, j = t / MR < ngr ? t / MR : 0;
+    const int t = w + W * i, j = t / MU < ngr ? t / MU : 0;
+    if constexpr (OP == PT_QKV) head_load<S>(group_params(pg, g0 + j), layer, rb0 / RU + t % MU, n, kg, hin[i]);
     if constexpr (NORM) {
       const float* q = advance(ssq_slot<S>(p0, 0, GU ? 1 : 0), j * gs) + n;
 #pragma unroll
       for (int e = 0; e < PER; ++e) sv[i][e] = q[(kg * PER + e) * BMAX];
     } else {
-      const int row = (rb0 + t % MR) * 16 + 4 * kg;
+      const int row = (rb0 + t % MU) * 16 + 4 * kg;
       xr[i] = *reinterpret_cast<const f32x4*>(advance(x_slot<S>(p0, 0, CI), j * gs) + x_at(n, row));
       gw[i] = *reinterpret_cast<const u32x2*>(gain + row);
     }
@@ -839,15 +946,18 @@ __global__ __launch_bounds__(T::W * kWave) void bk_pgemm(PGroup pg, int layer) {
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
-    const int t = w + W * i, j = t / MR, rb = rb0 + t % MR;
+    const int t = w + W * i, j = t / MU, rb = rb0 + t % MU * RU;
     if (t >= TL || j >= ngr) break;
-    f32x4 v[NB];
+    f32x4 v[RU][NB];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      v[b] = red[0][t][b][l];
+    for (int r = 0; r < RU; ++r)
 #pragma unroll
-      for (int k = 1; k < W; ++k) v[b] += red[k][t][b][l];
-    }
+      for (int b = 0; b < NB; ++b) {
+        const int e = j * MR + t % MU * RU + r;
+        v[r][b] = red[0][e][b][l];
+#pragma unroll
+        for (int k = 1; k < W; ++k) v[r][b] += red[k][e][b][l];
+      }
     const BParams p = group_params(pg, g0 + j);
     const bool on = n < p.B;
     const int row = rb * 16 + 4 * kg;
@@ -861,7 +971,7 @@ __global__ __launch_bounds__(T::W * kWave) void bk_pgemm(PGroup pg, int layer) {
         uint16_t h[4], o[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float g = v[0][e] * rs, u = v[NB - 1][e] * rs;
+          const float g = v[0][0][e] * rs, u = v[0][NB - 1][e] * rs;
           split2(g / (1.0f + __expf(-g)) * u, h[e], o[e]);  // SiLU(g) * u (reference utils.cuh:59-61)
         }
         if (on) {
@@ -870,10 +980,13 @@ __global__ __launch_bounds__(T::W * kWave) void bk_pgemm(PGroup pg, int layer) {
           st4(q + BMAX * S::F, o);
         }
       } else {
-        if (on) *reinterpret_cast<f32x4*>(qkv_slot<S>(p, 0) + (long long)n * S::QKV + row) = v[0] * rs;
+        f32x4 hv[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) hv[r] = v[r % RU][0] * rs;
+        qkv_head<S>(p, layer, rb / 4, n, kg, on, hin[i], hv);
       }
     } else {
-      f32x4 xn = xr[i] + v[0];
+      f32x4 xn = xr[i] + v[0][0];
       uint16_t h[4], o[4];
       float sq = 0.f;
 #pragma unroll
@@ -1006,48 +1119,6 @@ __global__ void bk_tok(BParams p) {
   }
   __syncthreads();
   if (b == 0) *p.step = s + 1;
-}
-
-// ------------------------------------------------------------ prefill
-// K / V of every column's position stored before the layer's attention reads
-// the cache: in a prefill the columns are consecutive prompt tokens of ONE
-// sequence (shared cache), and column b attends to the positions of columns
-// < b, which no bk_attn item of the same launch may still be writing.  Same
-// arithmetic as bk_attn's prologue: k = RoPE(k_norm(k)), both stored as bf16
-// (reference kv_cache.cuh:58-78).  One workgroup per (column, kv head): wave
-// 0 stores k, wave 1 stores v.
-template <class S, bool K8, class G>
-__global__ __launch_bounds__(2 * kWave) void bk_append(G pg, int layer) {
-  const BParams& p = group_of(pg);  // column group
-  // K8: FP8 rows (codes + the row's power-of-two scale from the wave's maximum)
-  static_assert(S::D == kWave, "one lane per head dimension");
-  constexpr int D = S::D, NKV = S::NKV;
-  const int b = blockIdx.x / NKV, g = blockIdx.x % NKV;
-  if (b >= p.B) return;
-  const int w = threadIdx.x / kWave, l = threadIdx.x % kWave;
-  const int pos = p.pos[b];
-  const long long kbase = (long long)b * p.kv_seq + ((long long)layer * NKV + g) * (long long)p.s_pad * D;
-  float v = qkv_slot<S>(p, 0)[(long long)b * S::QKV + (w == 0 ? S::QD + g * D : S::QD + S::KVD + g * D) + l];
-  if (w == 0) {
-    const float ss = wave_sum(v * v);
-    v = v * rsqrtf(ss / (float)D + kRmsEps) *
-        bf16_to_f32(p.norms[(long long)layer * S::NORM_STRIDE + S::NORM_K + l]);
-    const float partner = lane_xor32(v);
-    const int d = l & 31;
-    const float c = p.rope[(b * 2 + 0) * (D / 2) + d], sn = p.rope[(b * 2 + 1) * (D / 2) + d];
-    v = l < 32 ? v * c - partner * sn : v * c + partner * sn;
-  }
-  const long long at = w == 0 ? kbase + (long long)pos * D + l
-                              : kbase + (long long)(pos / 32) * 32 * D + (long long)l * 32 + (pos % 32);
-  if constexpr (K8) {
-    const int e = e4m3_row_exp(wave_max(fabsf(v)));
-    reinterpret_cast<uint8_t*>(w == 0 ? p.kv : p.kvt)[at] = (uint8_t)e4m3_encode(ldexpf(v, -e));
-    if (l == 0)
-      (w == 0 ? p.kscale : p.vscale)[(long long)b * p.sc_seq + ((long long)layer * NKV + g) * p.s_pad + pos] =
-          ldexpf(1.f, e);
-  } else {
-    (w == 0 ? p.kv : p.kvt)[at] = f32_to_bf16(v);
-  }
 }
 
 // ------------------------------------------------------------ attention
@@ -1237,7 +1308,7 @@ __device__ __forceinline__ bool attn_item(const BParams& p, int layer, int ep, A
     const int t0 = 32 * (s * AW * NBW + w + AW * q);
     if (t0 >= n) break;  // uniform over the wave (every block of an item that is off)
     // position pos takes K / V from LDS (this item appended them; in a
-    // prefill bk_append stored them before this kernel)
+    // prefill the QKV kernel stored them before this kernel)
     if (!p.prefill && pos >= t0 && pos < t0 + 32) {
       const int rp = pos - t0;
       if constexpr (K8) {
@@ -1547,12 +1618,10 @@ __global__ __launch_bounds__(PC_AW * kWave) void bk_pattn(PGroup pg, int layer) 
   static_assert(S::GQA == 2 && S::D == 64, "2 q heads of 64 per kv head");
   static_assert(NPART == 2 || NPART == 3, "two or three bf16 parts");
   constexpr int D = S::D, NKV = S::NKV, AWc = PC_AW, NT = PC_AW * kWave, QT = PC_NQ / 16;
-  constexpr int QP = D + 8;  // padded q row (elements)
   // q is multiplied by log2(e) / sqrt(D) before it is split, so a score is
   // already the exponent of 2 of its softmax weight
   constexpr float kLog2Scale = 1.4426950408889634f / 8.0f;
   static_assert(D == 64, "1 / sqrt(D) = 1 / 8");
-  __shared__ __attribute__((aligned(16))) uint16_t qs[NPART][PC_NQ][QP];
   __shared__ float ow[AWc][PC_NQ][D + 4];  // padded rows: the lanes of one store hit distinct banks
   __shared__ float mw[AWc][PC_NQ], lw[AWc][PC_NQ];
   // the longest prefixes (the last groups) first
@@ -1570,56 +1639,34 @@ __global__ __launch_bounds__(PC_AW * kWave) void bk_pattn(PGroup pg, int layer) 
   if (32 * w + 32 <= p.s_pad) pc_load<S, K8>(p, rk, rv, sbase, 32 * w, c16, gq, cur);
   __builtin_amdgcn_sched_barrier(0);
   const int p0 = p.pos[0], pmax = p0 + p.B - 1, nblk = pmax / 32 + 1;
-  // 1. q of the 32 queries (wave w: queries NQW w .. NQW w + NQW - 1; lane =
-  //    dimension): QK-norm (reference rmsnorm.cuh:57-84) and RoPE
-  //    rotate-half (attention.cuh:22-44), as bk_attn's prologue; every
-  //    query's loads are issued before the first is used
-  {
-    constexpr int NQW = PC_NQ / AWc;
-    const uint16_t* gn = p.norms + (long long)layer * S::NORM_STRIDE + S::NORM_Q;
-    const float gain = bf16_to_f32(gn[l]);
-    const int d = l & 31;
-    float qv[NQW], qc[NQW], qn[NQW];
-#pragma unroll
-    for (int k = 0; k < NQW; ++k) {
-      const int q = NQW * w + k, col = q >> 1, j = q & 1;
-      const bool on = col < p.B;
-      qv[k] = on ? qkv_slot<S>(p, 0)[(long long)col * S::QKV + (g * 2 + j) * D + l] : 0.f;
-      qc[k] = on ? p.rope[(col * 2 + 0) * (D / 2) + d] : 0.f;
-      qn[k] = on ? p.rope[(col * 2 + 1) * (D / 2) + d] : 0.f;
-    }
-#pragma unroll
-    for (int k = 0; k < NQW; ++k) {
-      const int q = NQW * w + k, col = q >> 1;
-      const bool on = col < p.B;
-      float v = qv[k];
-      const float ss = wave_sum(v * v);
-      v = on ? v * rsqrtf(ss / (float)D + kRmsEps) * gain : 0.f;
-      const float partner = lane_xor32(v);
-      const float cs = qc[k], sn = qn[k];
-      v = l < 32 ? v * cs - partner * sn : v * cs + partner * sn;
-      v *= kLog2Scale;  // scores in log2 units, softmax scale included
-      if constexpr (NPART == 3) {
-        uint16_t h, m, o;
-        split_bf16(v, h, m, o);
-        qs[0][q][l] = h, qs[1][q][l] = m, qs[2][q][l] = o;
-      } else {
-        uint32_t h, o;
-        bf16_hilo2(v, 0.f, h, o);
-        qs[0][q][l] = (uint16_t)h, qs[1][q][l] = (uint16_t)o;
-      }
-    }
-  }
-  __syncthreads();
-  // the q parts as B operands, held for the whole loop
+  // 1. the queries (normalised and rotated, qkv_head) as B operands, held for
+  //    the whole loop: lane (gq, c16) takes dims 32 kc + 8 gq .. + 7 of query
+  //    16 qt + c16 and splits them in registers
   u32x4 qb[QT][NPART][2];
+  {
+    f32x4 qv[QT][2][2];
 #pragma unroll
-  for (int qt = 0; qt < QT; ++qt)
-#pragma unroll
-    for (int pt = 0; pt < NPART; ++pt)
+    for (int qt = 0; qt < QT; ++qt) {
+      const int q = 16 * qt + (int)c16, col = q >> 1, j = q & 1;
+      const float* src = qkv_slot<S>(p, 0) + (long long)(col < p.B ? col : 0) * S::QKV + (g * 2 + j) * D + 8 * gq;
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc)
-        qb[qt][pt][kc] = *reinterpret_cast<const u32x4*>(&qs[pt][16 * qt + c16][32 * kc + 8 * gq]);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) qv[qt][kc][e] = *reinterpret_cast<const f32x4*>(src + 32 * kc + 4 * e);
+    }
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) {
+        float x[8];
+        u32x4 parts[NPART];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = qv[qt][kc][e / 4][e % 4] * kLog2Scale;  // log2 units, softmax scale included
+        pc_parts<NPART>(x, parts);
+#pragma unroll
+        for (int pt = 0; pt < NPART; ++pt) qb[qt][pt][kc] = parts[pt];
+      }
+  }
   // 2. the wave's blocks
   float m[QT], ls[QT];
   int qpos[QT];
