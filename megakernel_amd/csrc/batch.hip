@@ -3,6 +3,7 @@
 // the reference ABI; the kernels are in mk_batch.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -41,6 +42,7 @@ struct BHandle {
   // sizes), pf_gstride bytes apart, grown as prompts need more groups
   char* pf_slab = nullptr;
   int pf_groups = 0;
+  float* pf_part = nullptr;  // attention partials of a split prefix, shared by a pass's workgroups
   long long pf_gstride = 0;
 };
 
@@ -170,6 +172,20 @@ static void launch_pgemm_down(BHandle* h, const PGroup& g, int l) {
   else launch_pgemm<S, PT_DN, PTile<4, 4, 1, 2, 4>>(h, g, l);
 }
 
+// The attention of a prefill pass: eight waves per workgroup, and the prefix
+// in splits, where the (kv head, group) pairs leave CUs idle (PC_WG); four
+// waves, two workgroups per CU, where they do not.
+template <class S, bool K8>
+static void launch_pattn(BHandle* h, const PGroup& g, int l) {
+  const int wgs = S::NKV * g.n, nblk = (g.pos0 + g.ntok - 1) / 32 + 1;
+  if (wgs > PC_WG) {
+    hipLaunchKernelGGL((bk_pattn<S, K8, 4>), dim3(S::NKV, g.n), dim3(4 * kWave), 0, h->stream, g, l);
+    return;
+  }
+  int nz = std::min(std::min(PC_WG / wgs, PC_NZ), nblk / 16);
+  hipLaunchKernelGGL((bk_pattn<S, K8, 8>), dim3(S::NKV, g.n, nz < 1 ? 1 : nz), dim3(8 * kWave), 0, h->stream, g, l);
+}
+
 // One prefill pass: up to PG_MAX column groups of <= 16 consecutive prompt
 // tokens of one sequence (up to 1,024 tokens per pass over the weights):
 // the QKV kernel stores every column's K / V before the layer's attention; the
@@ -183,10 +199,8 @@ static int launch_prefill(BHandle* h, const PGroup& g, const BParams& pl, bool l
   hipLaunchKernelGGL((bk_embed<S, PGroup>), dim3(BMAX, ng), dim3(256), 0, h->stream, g);
   for (int l = 0; l < L; ++l) {
     launch_pgemm_qkv<S>(h, g, l);
-    if (p.kscale)
-      hipLaunchKernelGGL((bk_pattn<S, true>), dim3(S::NKV, ng), dim3(PC_AW * kWave), 0, h->stream, g, l);
-    else
-      hipLaunchKernelGGL((bk_pattn<S, false>), dim3(S::NKV, ng), dim3(PC_AW * kWave), 0, h->stream, g, l);
+    if (p.kscale) launch_pattn<S, true>(h, g, l);
+    else launch_pattn<S, false>(h, g, l);
     launch_pgemm_o<S>(h, g, l);
     launch_pgemm_gu<S>(h, g, l);
     launch_pgemm_down<S>(h, g, l);
@@ -440,9 +454,9 @@ static int run_steps(BHandle* h, const int* first, int n, int* out) {
 // block, in BParams order x, xg, ssq, qkv, att, act, part, cnt, gpart, gcnt,
 // keys, rope.
 static long long group_layout(const BHandle* h, long long off[12]) {
-  // the prefill kernels keep no attention partials or split-K sums (their
-  // attention merges in registers, their GEMMs run the whole K): part, cnt,
-  // gpart and gcnt get one line each
+  // the prefill kernels keep no split-K sums (their GEMMs run the whole K) and
+  // one partial buffer for all groups (pf_part): part, gpart and gcnt get one
+  // line each, cnt (finished prefix splits per kv head) too
   const long long sz[12] = {(long long)2 * BMAX * h->H * 4,
                             (long long)4 * BMAX * h->H * 2,
                             (long long)2 * (h->H / 16) * BMAX * 4,
@@ -480,6 +494,7 @@ static int ensure_groups(BHandle* h, int ng) {
     h->pf_slab = nullptr, h->pf_groups = 0;
   }
   if (alloc(h, &h->pf_slab, (size_t)stride * ng)) return -1;
+  if (!h->pf_part && alloc(h, &h->pf_part, (size_t)PC_WG * PC_PW * 4, false)) return -1;
   HIPCHK(hipStreamSynchronize(h->stream), -1);
   h->pf_groups = ng, h->pf_gstride = stride;
   return 0;
@@ -523,7 +538,7 @@ static int prefill_passes(BHandle* h, int seq, const int* tokens, int n, int pos
     pp.x = reinterpret_cast<float*>(slab + off[0]), pp.xg = reinterpret_cast<uint16_t*>(slab + off[1]);
     pp.ssq = reinterpret_cast<float*>(slab + off[2]), pp.qkv = reinterpret_cast<float*>(slab + off[3]);
     pp.att = reinterpret_cast<uint16_t*>(slab + off[4]), pp.act = reinterpret_cast<uint16_t*>(slab + off[5]);
-    pp.part = reinterpret_cast<float*>(slab + off[6]), pp.cnt = reinterpret_cast<int*>(slab + off[7]);
+    pp.part = h->pf_part, pp.cnt = reinterpret_cast<int*>(slab + off[7]);
     pp.gpart = reinterpret_cast<float*>(slab + off[8]), pp.gcnt = reinterpret_cast<int*>(slab + off[9]);
     pp.keys = reinterpret_cast<u64*>(slab + off[10]), pp.rope = reinterpret_cast<float*>(slab + off[11]);
     // every column writes and reads this sequence's cache (FP8: byte index =
@@ -548,6 +563,7 @@ static int prefill_passes(BHandle* h, int seq, const int* tokens, int n, int pos
     g.gstride = h->pf_gstride;
     g.n = (ntok + BMAX - 1) / BMAX;
     g.ntok = ntok;
+    g.pos0 = pos0 + c0;
     pp.B = ntok < BMAX ? ntok : BMAX;
     const bool last = ps == passes - 1;
     BParams pl = group_params(g, g.n - 1);

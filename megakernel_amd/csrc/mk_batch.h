@@ -141,6 +141,7 @@ struct PGroup {
   BParams p;
   long long gstride;
   int n, ntok;  // groups and tokens of the pass
+  int pos0;     // position of the pass's first token (group gi starts at pos0 + 16 gi)
 };
 
 template <class T>
@@ -1523,10 +1524,10 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(ATTN_WAVES_P
 }
 
 // ------------------------------------------------------------ prefill attention
-// One workgroup of PC_AW waves per (kv head g, column group): the group's
+// One workgroup of AWc waves per (kv head g, column group): the group's
 // <= 16 tokens x 2 q heads = 32 queries (query q: token q / 2, head 2 g + q % 2)
 // as two 16-column tiles; wave w takes the 32-position K / V blocks w, w +
-// PC_AW, ... of the causal prefix [0, the group's last position] with an
+// AWc, ... of the causal prefix [0, the group's last position] with an
 // online softmax per query, and the waves' states are combined at the end.
 // Products (v_mfma_f32_16x16x32_bf16):
 //   scores^T (16 positions x 16 queries) = K (A operand: the cache rows as
@@ -1549,8 +1550,13 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(ATTN_WAVES_P
 #ifndef MK_PATTN_NPART
 #define MK_PATTN_NPART 3
 #endif
-constexpr int PC_AW = 4;         // waves of a workgroup
 constexpr int PC_NQ = 2 * BMAX;  // queries of a workgroup (a column group x 2 q heads)
+// Prefix splits (grid z): with few column groups a workgroup per (kv head,
+// group) leaves most of the chip idle, so the prefix is cut into up to PC_NZ
+// splits while there are at most PC_WG workgroups, each with at least two
+// blocks per wave; the split that finishes last merges (as in bk_attn).
+constexpr int PC_WG = 256, PC_NZ = 16;
+constexpr int PC_PW = PC_NQ * 64 + 2 * PC_NQ;  // floats of a split's partial: o[32][64], max[32], sum[32]
 template <class S, bool K8>
 struct PcKV {  // one block's K / V operands of a lane, as loaded (K8: FP8 codes, converted at use)
   using Reg = typename std::conditional<K8, u32x2, u32x4>::type;
@@ -1613,11 +1619,11 @@ __device__ __forceinline__ void pc_parts(const float (&x)[8], u32x4 (&o)[NPART])
     }
   }
 }
-template <class S, bool K8, int NPART = MK_PATTN_NPART>
-__global__ __launch_bounds__(PC_AW * kWave) void bk_pattn(PGroup pg, int layer) {
+template <class S, bool K8, int AWc, int NPART = MK_PATTN_NPART>
+__global__ __launch_bounds__(AWc * kWave) void bk_pattn(PGroup pg, int layer) {
   static_assert(S::GQA == 2 && S::D == 64, "2 q heads of 64 per kv head");
   static_assert(NPART == 2 || NPART == 3, "two or three bf16 parts");
-  constexpr int D = S::D, NKV = S::NKV, AWc = PC_AW, NT = PC_AW * kWave, QT = PC_NQ / 16;
+  constexpr int D = S::D, NKV = S::NKV, NT = AWc * kWave, QT = PC_NQ / 16;
   // q is multiplied by log2(e) / sqrt(D) before it is split, so a score is
   // already the exponent of 2 of its softmax weight
   constexpr float kLog2Scale = 1.4426950408889634f / 8.0f;
@@ -1625,20 +1631,21 @@ __global__ __launch_bounds__(PC_AW * kWave) void bk_pattn(PGroup pg, int layer) 
   __shared__ float ow[AWc][PC_NQ][D + 4];  // padded rows: the lanes of one store hit distinct banks
   __shared__ float mw[AWc][PC_NQ], lw[AWc][PC_NQ];
   // the longest prefixes (the last groups) first
-  const BParams p = group_params(pg, pg.n - 1 - (int)blockIdx.y);
+  const int gi = pg.n - 1 - (int)blockIdx.y;
+  const BParams p = group_params(pg, gi);
   const int g = blockIdx.x, tid = ltid(), w = wave_id(), l = (int)lane_id();
   const unsigned c16 = (unsigned)l & 15u, gq = (unsigned)l >> 4;
   const long long kbase = ((long long)layer * NKV + g) * (long long)p.s_pad * D;
   const long long sbase = ((long long)layer * NKV + g) * p.s_pad;
   const auto rk = K8 ? make_rsrc(reinterpret_cast<const uint8_t*>(p.kv) + kbase) : make_rsrc(p.kv + kbase);
   const auto rv = K8 ? make_rsrc(reinterpret_cast<const uint8_t*>(p.kvt) + kbase) : make_rsrc(p.kvt + kbase);
-  // the wave's first block is loading during the prologue, issued before the
-  // group's position is read (block w lies inside the cache whatever the
-  // prefix; unused when the prefix is shorter)
+  const int p0 = pg.pos0 + BMAX * gi, pmax = p0 + p.B - 1, nall = pmax / 32 + 1;
+  // this split's blocks [b0, nblk) of the prefix; the wave's first one is
+  // loading during the prologue
+  const int nz = gridDim.z, z = blockIdx.z, b0 = z * nall / nz, nblk = (z + 1) * nall / nz;
   PcKV<S, K8> cur, nxt;
-  if (32 * w + 32 <= p.s_pad) pc_load<S, K8>(p, rk, rv, sbase, 32 * w, c16, gq, cur);
+  if (b0 + w < nblk) pc_load<S, K8>(p, rk, rv, sbase, 32 * (b0 + w), c16, gq, cur);
   __builtin_amdgcn_sched_barrier(0);
-  const int p0 = p.pos[0], pmax = p0 + p.B - 1, nblk = pmax / 32 + 1;
   // 1. the queries (normalised and rotated, qkv_head) as B operands, held for
   //    the whole loop: lane (gq, c16) takes dims 32 kc + 8 gq .. + 7 of query
   //    16 qt + c16 and splits them in registers
@@ -1756,7 +1763,7 @@ __global__ __launch_bounds__(PC_AW * kWave) void bk_pattn(PGroup pg, int layer) 
   // paths, also waited for the block after.
   // The scheduling barriers keep the loads where they are: the scheduler
   // otherwise sinks them to their first use.
-  for (int kb = w; kb < nblk; kb += 2 * AWc) {
+  for (int kb = b0 + w; kb < nblk; kb += 2 * AWc) {
     pc_load<S, K8>(p, rk, rv, sbase, 32 * min(kb + AWc, nblk - 1), c16, gq, nxt);
     __builtin_amdgcn_sched_barrier(0);
     block(32 * kb, cur);
@@ -1780,34 +1787,82 @@ __global__ __launch_bounds__(PC_AW * kWave) void bk_pattn(PGroup pg, int layer) 
     }
   }
   __syncthreads();
-  {  // thread: 8 dims of one query, one 16-byte store per plane
-    static_assert(NT * 8 == PC_NQ * D, "eight outputs per thread");
-    const int q = tid / (D / 8), d0 = tid % (D / 8) * 8, col = q >> 1, j = q & 1;
-    if (col >= p.B) return;
-    float M = mw[0][q];
+  // thread: OD dims of one query
+  constexpr int OD = PC_NQ * D / NT;
+  static_assert(OD == 4 || OD == 8, "whole 8-byte stores per thread");
+  const int q = tid / (D / OD), d0 = tid % (D / OD) * OD, col = q >> 1, j = q & 1;
+  float M = mw[0][q], o[OD], L = 0.f;
 #pragma unroll
-    for (int i = 1; i < AWc; ++i) M = fmaxf(M, mw[i][q]);
-    float o[8], L = 0.f;
+  for (int i = 1; i < AWc; ++i) M = fmaxf(M, mw[i][q]);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = 0.f;
+  for (int e = 0; e < OD; ++e) o[e] = 0.f;
 #pragma unroll
-    for (int i = 0; i < AWc; ++i) {
-      const float f = mw[i][q] == -INFINITY ? 0.f : exp2f(mw[i][q] - M);
+  for (int i = 0; i < AWc; ++i) {
+    const float f = mw[i][q] == -INFINITY ? 0.f : exp2f(mw[i][q] - M);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = fmaf(f, ow[i][q][d0 + e], o[e]);
-      L = fmaf(f, lw[i][q], L);
+    for (int e = 0; e < OD; ++e) o[e] = fmaf(f, ow[i][q][d0 + e], o[e]);
+    L = fmaf(f, lw[i][q], L);
+  }
+  if (nz > 1) {
+    // the split's partial, written through and acknowledged before it is
+    // counted; the last split of (group, kv head) adds them in split order
+    __shared__ int last;
+    float* part = pg.p.part + (long long)(gi * NKV + g) * nz * PC_PW;
+    {
+      float* mine = part + (long long)z * PC_PW;
+#pragma unroll
+      for (int e = 0; e < OD; ++e)
+        __hip_atomic_store(mine + q * D + d0 + e, o[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (d0 == 0) {
+        __hip_atomic_store(mine + PC_NQ * D + q, M, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(mine + PC_NQ * D + PC_NQ + q, L, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
     }
-    u32x4 hi, lo;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      uint16_t h0, l0, h1, l1;
-      split2(o[2 * e] / L, h0, l0);
-      split2(o[2 * e + 1] / L, h1, l1);
-      hi[e] = h0 | (unsigned)h1 << 16, lo[e] = l0 | (unsigned)l1 << 16;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+      const int done = __hip_atomic_fetch_add(p.cnt + g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = done == nz - 1;
+      if (last) __hip_atomic_store(p.cnt + g, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next layer
     }
-    uint16_t* a = att_slot<S>(p, 0) + unit_at(col, (g * 2 + j) * D + d0);
-    *reinterpret_cast<u32x4*>(a) = hi;
-    *reinterpret_cast<u32x4*>(a + BMAX * S::QD) = lo;
+    __syncthreads();
+    if (!last) return;
+    float mv[PC_NZ], lv[PC_NZ], ov[PC_NZ][OD];  // every split's loads before the first use
+#pragma unroll
+    for (int k = 0; k < PC_NZ; ++k) {
+      const float* pk = part + (long long)(k < nz ? k : 0) * PC_PW;
+      if (k < nz) {
+        mv[k] = __hip_atomic_load(pk + PC_NQ * D + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lv[k] = __hip_atomic_load(pk + PC_NQ * D + PC_NQ + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int e = 0; e < OD; ++e)
+          ov[k][e] = __hip_atomic_load(pk + q * D + d0 + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int k = 0; k < PC_NZ; ++k) M = k < nz ? fmaxf(M, mv[k]) : M;
+#pragma unroll
+    for (int e = 0; e < OD; ++e) o[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < PC_NZ; ++k) {
+      if (k < nz) {
+        const float f = mv[k] == -INFINITY ? 0.f : exp2f(mv[k] - M);
+#pragma unroll
+        for (int e = 0; e < OD; ++e) o[e] = fmaf(f, ov[k][e], o[e]);
+        L = fmaf(f, lv[k], L);
+      }
+    }
+  }
+  if (col >= p.B) return;
+  uint16_t* a = att_slot<S>(p, 0) + unit_at(col, (g * 2 + j) * D + d0);
+#pragma unroll
+  for (int c = 0; c < OD; c += 4) {
+    uint16_t hi[4], lo[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split2(o[c + e] / L, hi[e], lo[e]);
+    st4(a + c, hi);
+    st4(a + BMAX * S::QD + c, lo);
   }
 }
 

@@ -653,3 +653,32 @@ def test_prefill_tile_shapes_agree(which):
     finally:
         eng.close()
         dw.free()
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+@pytest.mark.parametrize("prefix,n", [(480, 3), (1000, 20), (2047, 1), (4100, 17), (8300, 2), (3000, 260)])
+def test_prefill_split_prefix_equals_decode(prefix, n, kv8):
+    """Prefill attention with its prefix in one to sixteen splits (few column
+    groups behind a long cache; 260 tokens: 17 groups, one split) against the
+    decode step's attention, token by token on the same cache.  fp32 logits
+    within 1e-3 of their RMS; with FP8 rows, whose roundings to 3 bits may fall
+    the other way, within 1e-2."""
+    shape = BASELINE.with_(n_layers=2, vocab=4096)
+    dw = DeviceWeights(shape, 6, gain_std=0.1)
+    eng = BatchEngine(dw, 1, prefix + n + 8, shape)
+    try:
+        eng.set_kv_fp8(kv8)
+        eng.fill_kv_synthetic(0, prefix, 21)
+        prompt = [(53 * i * i + 7 * i + 1) % shape.vocab for i in range(n)]
+        for t in prompt[:-1]:
+            eng.decode([t])
+        _, want = eng.debug_logits(prompt[-1:])
+        for _ in range(2):  # twice: the splits' counters are re-armed
+            eng.set_pos(0, prefix)
+            _, got = eng.prefill(0, prompt, with_logits=True)
+            rms = float(np.sqrt(np.mean(want[0].astype(np.float64) ** 2)))
+            err = float(np.abs(got - want[0]).max()) / rms
+            assert err < (1e-2 if kv8 else 1e-3), f"logits off by {err:.2e} of their RMS"
+    finally:
+        eng.close()
+        dw.free()
