@@ -1540,13 +1540,18 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(ATTN_WAVES_P
 // end, and the weights never pass through LDS.  NPART 3: q and the weights
 // split exactly (hi + mid + lo by truncation); 2: hi + lo (RNE), relative
 // error <= 2^-17.
-// (measured per layer at 1,024 tokens, us: 8 waves 22.6 against 4 waves
-// 20.9; three K / V register sets 23.2 against two 20.6; two parts 20.8
-// against three 21.6; a timing probe limited to one block per workgroup
-// 9.0, so about half is the prologue, the merge and the launch; the earlier
-// kernel with q
-// as the A operand -- 4 queries per 16-row tile, the weights through LDS --
-// 34.0.)
+// The score tiles take the positions of a block in the order 8 (r / 4) + 4 h +
+// r % 4 (row r of tile h), so a lane's eight weights are eight consecutive
+// positions and V^T is read 16 bytes at a time.
+// What bounds it: the vector work beside the products (about 1,000 cycles of
+// softmax and splitting per block step against 768 of matrix products) and,
+// for a few groups, the load round trip of a wave's next block; two waves per
+// SIMD.  us per layer, 64 groups at position 0 / 1,024 / 3,072: 19.1 / 34.5 /
+// 63.7 with 8-byte V loads, non-temporal loads and one query tile after the
+// other, 15.2 / 27.0 / 50.5 as it is; FP8 23.7 / 43.5 / 82.7 and 16.3 / 30.4 /
+// 57.1; 13 groups at 1,500: 17.0 and 14.7.
+// (Earlier measurements: three K / V register sets 23.2 against two 20.6; two
+// parts 20.8 against three 21.6.)
 #ifndef MK_PATTN_NPART
 #define MK_PATTN_NPART 3
 #endif
@@ -1561,8 +1566,8 @@ template <class S, bool K8>
 struct PcKV {  // one block's K / V operands of a lane, as loaded (K8: FP8 codes, converted at use)
   using Reg = typename std::conditional<K8, u32x2, u32x4>::type;
   Reg k[2][2];  // [16-position half][32-dim chunk]
-  Reg v[S::D / 16];  // [16-dim tile]: positions (4 gq .. 4 gq + 3, 16 + 4 gq .. 16 + 4 gq + 3)
-  f32x4 sk[2], sv[2];  // K8: row scales of the lane's score positions t0 + 16 h + 4 gq + i
+  Reg v[S::D / 16];  // [16-dim tile]: positions 8 gq .. 8 gq + 7
+  f32x4 sk[2], sv[2];  // K8: row scales of the lane's score positions t0 + 8 gq + 4 h + i
 };
 // bf16 operand of a loaded register: FP8 codes converted exactly (scale 1)
 __device__ __forceinline__ u32x4 pc_op(u32x4 r) { return r; }
@@ -1575,29 +1580,25 @@ __device__ __forceinline__ void pc_load(const BParams& p, __amdgpu_buffer_rsrc_t
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc) {
-      const unsigned e = ((unsigned)t0 + 16u * h + c16) * D + 32u * kc + 8u * gq;
+      const unsigned e = ((unsigned)t0 + 8u * (c16 >> 2) + 4u * h + (c16 & 3u)) * D + 32u * kc + 8u * gq;
       if constexpr (K8)
-        r.k[h][kc] = __builtin_amdgcn_raw_buffer_load_b64(rk, e, 0u, 2);
+        r.k[h][kc] = __builtin_amdgcn_raw_buffer_load_b64(rk, e, 0u, 0);
       else
-        r.k[h][kc] = __builtin_amdgcn_raw_buffer_load_b128(rk, e * 2u, 0u, 2);
+        r.k[h][kc] = __builtin_amdgcn_raw_buffer_load_b128(rk, e * 2u, 0u, 0);
     }
 #pragma unroll
   for (int dt = 0; dt < D / 16; ++dt) {
-    const unsigned e = (unsigned)t0 * D + (16u * dt + c16) * 32u + 4u * gq;
-    if constexpr (K8) {
-      r.v[dt] = u32x2{__builtin_amdgcn_raw_buffer_load_b32(rv, e, 0u, 2),
-                      __builtin_amdgcn_raw_buffer_load_b32(rv, e + 16u, 0u, 2)};
-    } else {
-      const u32x2 a = __builtin_amdgcn_raw_buffer_load_b64(rv, e * 2u, 0u, 2);
-      const u32x2 b = __builtin_amdgcn_raw_buffer_load_b64(rv, (e + 16u) * 2u, 0u, 2);
-      r.v[dt] = u32x4{a[0], a[1], b[0], b[1]};
-    }
+    const unsigned e = (unsigned)t0 * D + (16u * dt + c16) * 32u + 8u * gq;
+    if constexpr (K8)
+      r.v[dt] = __builtin_amdgcn_raw_buffer_load_b64(rv, e, 0u, 0);
+    else
+      r.v[dt] = __builtin_amdgcn_raw_buffer_load_b128(rv, e * 2u, 0u, 0);
   }
   if constexpr (K8) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      r.sk[h] = *reinterpret_cast<const f32x4*>(p.kscale + sbase + t0 + 16 * h + 4 * (int)gq);
-      r.sv[h] = *reinterpret_cast<const f32x4*>(p.vscale + sbase + t0 + 16 * h + 4 * (int)gq);
+      r.sk[h] = *reinterpret_cast<const f32x4*>(p.kscale + sbase + t0 + 8 * (int)gq + 4 * h);
+      r.sv[h] = *reinterpret_cast<const f32x4*>(p.vscale + sbase + t0 + 8 * (int)gq + 4 * h);
     }
   }
 }
@@ -1620,7 +1621,7 @@ __device__ __forceinline__ void pc_parts(const float (&x)[8], u32x4 (&o)[NPART])
   }
 }
 template <class S, bool K8, int AWc, int NPART = MK_PATTN_NPART>
-__global__ __launch_bounds__(AWc * kWave) void bk_pattn(PGroup pg, int layer) {
+__global__ __launch_bounds__(AWc * kWave) __attribute__((amdgpu_waves_per_eu(2))) void bk_pattn(PGroup pg, int layer) {
   static_assert(S::GQA == 2 && S::D == 64, "2 q heads of 64 per kv head");
   static_assert(NPART == 2 || NPART == 3, "two or three bf16 parts");
   constexpr int D = S::D, NKV = S::NKV, NT = AWc * kWave, QT = PC_NQ / 16;
@@ -1686,74 +1687,86 @@ __global__ __launch_bounds__(AWc * kWave) void bk_pattn(PGroup pg, int layer) {
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) acc[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  // the first position of a tile's queries when all its 8 tokens exist, else
-  // -1: a block that ends at or before it is visible to every query of the
-  // tile (no mask)
-  int qmin[QT];
-#pragma unroll
-  for (int qt = 0; qt < QT; ++qt) qmin[qt] = 8 * qt + 7 < p.B ? p0 + 8 * qt : -1;
-  // one query tile's products and online-softmax step on a block (r: its K /
-  // V operands); MASK: the causal mask and the guards of a query that has no
-  // visible position yet
-  const auto step = [&](auto mask_c, int qt, int t0, const PcKV<S, K8>& r) __attribute__((always_inline)) {
+  // the first query's position when all 16 tokens exist, else -1: a block
+  // that ends at or before it is visible to every query (no mask)
+  const int qmin = p.B == BMAX ? p0 : -1;
+  // the products and online-softmax step of both query tiles on a block (r:
+  // its K / V operands), in one straight line so that one tile's vector work
+  // runs beside the other's products; MASK: the causal mask and the guards of
+  // a query that has no visible position yet
+  const auto step = [&](auto mask_c, int t0, const PcKV<S, K8>& r) __attribute__((always_inline)) {
     constexpr bool MASK = decltype(mask_c)::value;
-    float sc[2][4];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      f32x4 d4 = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kc = 0; kc < 2; ++kc)
-#pragma unroll
-        for (int pt = 0; pt < NPART; ++pt) d4 = mfma(pc_op(r.k[h][kc]), qb[qt][pt][kc], d4);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // K8: the K row scale (a power of two) multiplies the exact product
-        const float x = K8 ? d4[i] * r.sk[h][i] : d4[i];
-        sc[h][i] = MASK && t0 + 16 * h + 4 * (int)gq + i > qpos[qt] ? -INFINITY : x;
-      }
-    }
-    float bm = fmaxf(fmaxf(fmaxf(sc[0][0], sc[0][1]), fmaxf(sc[0][2], sc[0][3])),
-                     fmaxf(fmaxf(sc[1][0], sc[1][1]), fmaxf(sc[1][2], sc[1][3])));
-    bm = max_xor32(max_xor16(bm));
-    const float mo = m[qt], mn = fmaxf(mo, bm);
-    m[qt] = mn;
-    float pw[8], ps = 0.f;
+    float sc[QT][2][4], mo[QT], mn[QT];
+    f32x4 d4[QT][2];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        // a query none of whose positions so far is visible keeps m = -inf
-        // and weight 0 (no -inf - -inf)
-        const float e = MASK && mn == -INFINITY ? 0.f : exp2f(sc[h][i] - mn);
-        ps += e;
-        pw[4 * h + i] = K8 ? e * r.sv[h][i] : e;  // the V row scale enters the weight
+      for (int kc = 0; kc < 2; ++kc) {
+        const u32x4 ka = pc_op(r.k[h][kc]);
+#pragma unroll
+        for (int pt = 0; pt < NPART; ++pt)
+#pragma unroll
+          for (int qt = 0; qt < QT; ++qt)
+            d4[qt][h] = mfma(ka, qb[qt][pt][kc], kc + pt == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : d4[qt][h]);
       }
+    bool grew = false;
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          // K8: the K row scale (a power of two) multiplies the exact product
+          const float x = K8 ? d4[qt][h][i] * r.sk[h][i] : d4[qt][h][i];
+          sc[qt][h][i] = MASK && t0 + 8 * (int)gq + 4 * h + i > qpos[qt] ? -INFINITY : x;
+        }
+      float bm = fmaxf(fmaxf(fmaxf(sc[qt][0][0], sc[qt][0][1]), fmaxf(sc[qt][0][2], sc[qt][0][3])),
+                       fmaxf(fmaxf(sc[qt][1][0], sc[qt][1][1]), fmaxf(sc[qt][1][2], sc[qt][1][3])));
+      bm = max_xor32(max_xor16(bm));
+      mo[qt] = m[qt], mn[qt] = fmaxf(m[qt], bm);
+      m[qt] = mn[qt];
+      grew |= mn[qt] != mo[qt];
+    }
     // the running state is rescaled only when some query's maximum grew (the
     // factor is exactly 1 otherwise).  The branch is taken by the whole wave:
     // a query still without a visible position (mn = mo = -inf) keeps factor
     // 1, not exp2(-inf - -inf)
-    if (__builtin_amdgcn_ballot_w64(mn != mo)) {
-      const float alpha = MASK && mn == -INFINITY ? 1.f : exp2f(mo - mn);
-      ls[qt] *= alpha;
+    if (__builtin_amdgcn_ballot_w64(grew)) {
 #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt)
+      for (int qt = 0; qt < QT; ++qt) {
+        const float alpha = MASK && mn[qt] == -INFINITY ? 1.f : exp2f(mo[qt] - mn[qt]);
+        ls[qt] *= alpha;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[qt][dt][i] *= alpha;
+        for (int dt = 0; dt < D / 16; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[qt][dt][i] *= alpha;
+      }
     }
-    ls[qt] += ps;
-    u32x4 pb[NPART];
-    pc_parts<NPART>(pw, pb);
-#pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt)
-#pragma unroll
-      for (int pt = 0; pt < NPART; ++pt) acc[qt][dt] = mfma(pc_op(r.v[dt]), pb[pt], acc[qt][dt]);
-  };
-  const auto block = [&](int t0, const PcKV<S, K8>& r) __attribute__((always_inline)) {
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
-      if (t0 + 31 <= qmin[qt]) step(std::false_type{}, qt, t0, r);
-      else step(std::true_type{}, qt, t0, r);
+      float pw[8], ps = 0.f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          // a query none of whose positions so far is visible keeps m = -inf
+          // and weight 0 (no -inf - -inf)
+          const float e = MASK && mn[qt] == -INFINITY ? 0.f : exp2f(sc[qt][h][i] - mn[qt]);
+          ps += e;
+          pw[4 * h + i] = K8 ? e * r.sv[h][i] : e;  // the V row scale enters the weight
+        }
+      ls[qt] += ps;
+      u32x4 pb[NPART];
+      pc_parts<NPART>(pw, pb);
+#pragma unroll
+      for (int pt = 0; pt < NPART; ++pt)
+#pragma unroll
+        for (int dt = 0; dt < D / 16; ++dt) acc[qt][dt] = mfma(pc_op(r.v[dt]), pb[pt], acc[qt][dt]);
     }
+  };
+  const auto block = [&](int t0, const PcKV<S, K8>& r) __attribute__((always_inline)) {
+    if (t0 + 31 <= qmin) step(std::false_type{}, t0, r);
+    else step(std::true_type{}, t0, r);
   };
   // two register sets in turn (no copy between them: a copy would wait for
   // the next block's loads before the current block's products).  Every
