@@ -588,3 +588,44 @@ def test_qwen3_class_kernel_equals_spread(ctx):
     finally:
         eng.close()
         dw.free()
+
+
+@pytest.mark.parametrize("kv8", [False, True])
+def test_reset_clears_every_written_row(kv8):
+    """reset zeroes the cache up to the highest row written since the last
+    clear, whichever path wrote it, at block edges and at the capacity; a
+    change of format clears what the other format held."""
+    shape = TINY
+    dw = DeviceWeights(shape, 3)
+    eng = MegakernelEngine(shape=shape, max_seq=96, device_weights=dw, prefill=True)
+    try:
+        eng.set_kv_fp8(kv8)
+
+        def fill(n):
+            eng.fill_kv_synthetic(n, 4)
+
+        def decode_past(n):
+            eng.set_pos(n - 3)
+            eng.decode_many(1, 3)
+            eng.set_pos(0)
+
+        def prefill_past(n):
+            eng.set_pos(n - 5)
+            eng.prefill([1, 2, 3, 4, 5])
+            eng.set_pos(2)
+
+        def set_kv(n):
+            eng.set_kv(np.full((shape.n_layers, 2, shape.n_kv_heads, n, shape.head_dim), 0x3F80, np.uint16))
+
+        for write in (fill, decode_past, prefill_past, set_kv):
+            for n in (7, 32, 33, 96):
+                write(n)
+                assert eng.get_kv(96)[:, :, :, n - 1].any()
+                eng.reset()
+                assert eng.pos == 0 and not eng.get_kv(96).any()
+        fill(96)
+        eng.set_kv_fp8(not kv8)
+        assert not eng.get_kv(96).any()
+    finally:
+        eng.close()
+        dw.free()
