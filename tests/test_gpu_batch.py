@@ -365,7 +365,7 @@ def test_batch_fp8_kv_16_sequences():
 
 def test_batch_fp8_kv_fill_exact_and_prefill():
     """FP8 fills bit-exact against the oracle; a prompt prefilled into an FP8
-    cache (bk_append quantising each row) gives the oracle's next token and
+    cache (the QKV kernel quantising each row) gives the oracle's next token and
     logits on the same dequantised cache, and leaves the other sequences'
     caches untouched."""
     lengths = [0, 40, 129]
