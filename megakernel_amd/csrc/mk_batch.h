@@ -715,9 +715,9 @@ __global__ __launch_bounds__(GT) void bk_down(G p, int layer) {
 // accumulator), NBUF chunks of CW units in flight.  The waves' sums meet in
 // LDS once, in wave order, and each wave runs the epilogue of its share of the
 // tiles: QKV scales by the group's norm factor and finishes whole heads
-// (qkv_head), gate / up applies SiLU, O and down add the residual and publish x (the next norm's parts and per-block
-// sums of squares) as publish_x does; the epilogue's inputs are loaded before
-// the product.
+// (qkv_head), gate / up applies SiLU, O and down add the residual and publish
+// x (the next norm's parts and per-block sums of squares) as publish_x does;
+// the epilogue's inputs are loaded before the product.
 //
 // What bounds it: a short pass the latency of one load round per kernel (23
 // tokens: 4 - 6 us per GEMM, a kernel's fixed cost about 4), a long one the
