@@ -329,11 +329,15 @@ def test_error_paths():
 
 @pytest.mark.parametrize("chunk,merge", [(64, None), (32, 4)])
 def test_qwen3_preset_head_dim_128(chunk, merge):
-    """The reference's own config.cuh shapes (head_dim 128, ffn 3072); chunk 32
-    gives 10 splits, merged by the first split's workgroup (merge threshold 4)."""
+    """The reference's own config.cuh shapes (head_dim 128, ffn 3072) in the
+    spread kernel, which keeps the chunk it is given (the automatic choice
+    would widen it to four splits for the class kernel): chunk 64 gives 5
+    splits, chunk 32 gives 10, merged by the first split's workgroup (merge
+    threshold 4)."""
     shape = QWEN3_06B.with_(n_layers=2, vocab=2048)
     eng, orc, dw = make_pair(shape, 31, 400)
     try:
+        eng.set_decode_kernel(_lib.KERNEL_SPREAD)
         eng.set_attention_chunk(chunk)
         if merge is not None:
             eng.set_attention_merge(merge)
