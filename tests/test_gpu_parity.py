@@ -9,6 +9,7 @@ tie-break.
 from __future__ import annotations
 
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -633,3 +634,31 @@ def test_reset_clears_every_written_row(kv8):
     finally:
         eng.close()
         dw.free()
+
+
+def test_reset_of_a_full_cache_keeps_the_memset_rate():
+    """A reset after the whole default capacity was written takes no longer than
+    a fill of the whole cache allocation (1.9 GB), give or take a fifth."""
+    shape = BASELINE.with_(vocab=4096)
+    dw = DeviceWeights(shape, 3)
+    eng = MegakernelEngine(shape=shape, max_seq=33024, device_weights=dw)
+    dw.free()
+    ref = torch.empty(2 * shape.n_layers * shape.n_kv_heads * 33024 * shape.head_dim, dtype=torch.int16, device="cuda")
+    try:
+        def us(work):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            work()
+            torch.cuda.synchronize()
+            return (time.perf_counter() - t) * 1e6
+
+        fills, resets = [], []
+        for _ in range(8):
+            eng.fill_kv_synthetic(33024, 7)
+            resets.append(us(eng.reset))
+            fills.append(us(ref.zero_))
+        print(f"reset {min(resets):.0f} us, fill of the allocation {min(fills):.0f} us", flush=True)
+        assert min(resets) < 1.2 * min(fills)
+        assert not eng.get_kv(64).any()
+    finally:
+        eng.close()
