@@ -19,6 +19,7 @@
 #include "mk_host.h"
 #include "mk_kernel.h"
 #include "mk_launch.h"
+#include "mk_written.h"
 
 #include "../../include/megakernel.h"
 
@@ -460,7 +461,7 @@ struct Handle {
   unsigned tag_base = 1;  // tag of the next launch's first phase (0 never valid)
   int pos = 0;
   long long kv_bytes = 0;
-  int kv_high = 0;             // no cache row at or past this position has been written since it was cleared
+  WrittenRows written;         // cache rows written since they were last cleared
   int s_pad = 0;               // KV capacity rounded up to whole 32-position blocks
   uint16_t* kvt = nullptr;     // V^T region inside the kv allocation
   DecodeLaunch launch = nullptr;
@@ -719,22 +720,25 @@ __global__ __launch_bounds__(kClearNT) void clear_rows_kernel(u32x4* __restrict_
 // 0.30 ms of every request's reset, of which a 150-token prompt and its
 // answer have written 9 MB (reset: 25 us).
 static void clear_cache(Handle* h) {
-  const long long hi = (h->kv_high + 31) / 32 * 32, rows = (long long)h->L * h->sh.NKV;
-  const auto clear = [&](void* base, long long unit) {  // unit: bytes per position of a row
-    const long long n = hi * unit / 16;
-    if (n > 0)
-      hipLaunchKernelGGL(clear_rows_kernel,
-                         dim3((unsigned)((n + kClearNT - 1) / kClearNT), (unsigned)std::min(rows, 65535LL)),
-                         dim3(kClearNT), 0, h->stream, static_cast<u32x4*>(base), h->s_pad * unit / 16, n, (int)rows);
-  };
-  const long long unit = h->sh.D * (h->kv_fp8 ? 1 : 2);
-  clear(h->kv, unit);
-  clear(h->kvt, unit);
-  if (h->kv_fp8) {
-    clear(h->kscale, 4);
-    clear(h->vscale, 4);
-  }
-  h->kv_high = 0;
+  const int rows = h->L * h->sh.NKV;
+  const bool done = h->written.clear([&](long long hi) {
+    bool ok = true;
+    const auto clear = [&](void* base, long long unit) {  // unit: bytes per position of a row
+      const long long n = hi * unit / 16;
+      hipLaunchKernelGGL(clear_rows_kernel, dim3((unsigned)((n + kClearNT - 1) / kClearNT), std::min(rows, 65535)),
+                         dim3(kClearNT), 0, h->stream, static_cast<u32x4*>(base), h->s_pad * unit / 16, n, rows);
+      ok = hipGetLastError() == hipSuccess && ok;
+    };
+    const long long unit = h->sh.D * (h->kv_fp8 ? 1 : 2);
+    clear(h->kv, unit);
+    clear(h->kvt, unit);
+    if (h->kv_fp8) {
+      clear(h->kscale, 4);
+      clear(h->vscale, 4);
+    }
+    return ok;
+  });
+  if (!done) set_err("reset: the cache could not be cleared");
 }
 
 // The attention chunk of a launch whose last token sits at position end - 1:
@@ -815,7 +819,7 @@ static int run(Handle* h, int first_token, int n, int* out_host, bool debug, int
     if (clear_pair_words(h)) return -1;
     h->chunk_eff = chunk;
   }
-  h->kv_high = std::max(h->kv_high, h->pos + n);
+  h->written.wrote(h->pos + n);
   p.chunk_min = chunk;
   p.merge_min = h->merge_min;
   p.pace_pct = h->pace_pct;
@@ -1137,7 +1141,7 @@ int megakernel_set_kv(void* handle, const void* host_kv, int len) {
     mk::set_err("invalid set_kv arguments (len %d)", len);
     return -1;
   }
-  h->kv_high = std::max(h->kv_high, len);
+  h->written.wrote(len);
   if (len > 0 && kv_transfer(h, const_cast<void*>(host_kv), len, 1)) return -1;
   if (mk::clear_pair_words(h)) return -1;
   h->pos = len;
@@ -1160,7 +1164,7 @@ int megakernel_fill_kv_synthetic(void* handle, int len, unsigned long long seed,
     mk::set_err("invalid fill_kv arguments (len %d)", len);
     return -1;
   }
-  h->kv_high = std::max(h->kv_high, len);
+  h->written.wrote(len);
   if (len > 0 && h->kv_fp8) {  // the bf16 values in the reference layout, then quantised rows
     const float c = (float)(std * sqrt(3.0) / 65536.0);
     void* stage = nullptr;
@@ -1258,7 +1262,7 @@ int megakernel_prefill(void* handle, const int* tokens, int n, int* next_token) 
     return -1;
   }
   // (clamped: a prompt past the capacity is refused below)
-  h->kv_high = std::max(h->kv_high, (int)std::min((long long)h->S, (long long)h->pos + std::max(n, 0)));
+  h->written.wrote((int)std::min((long long)h->S, (long long)h->pos + std::max(n, 0)));
   if (mk::batch::prefill_context_run(h->prefill, tokens, n, h->pos, next_token, nullptr,
                                      h->kv_fp8 ? h->kscale : nullptr, h->kv_fp8 ? h->vscale : nullptr)) return -1;
   h->pos += n;
@@ -1420,15 +1424,17 @@ int megakernel_set_kv_fp8(void* handle, int enable) {
     HIPCHK(hipMalloc(&h->kscale, sb), -1);
     HIPCHK(hipMalloc(&h->vscale, sb), -1);
   }
+  // a new, empty cache in the chosen format: whatever the other one held (every
+  // row counts as written until the whole allocation's clear is issued)
+  h->written.wrote(h->S);
   h->kv_fp8 = enable != 0;
-  // a new, empty cache in the chosen format: whatever the other one held
   HIPCHK(hipMemsetAsync(h->kv, 0, h->kv_bytes, h->stream), -1);
   if (h->kscale) {
     const size_t sb = (size_t)h->L * h->sh.NKV * h->s_pad * 4;
     HIPCHK(hipMemsetAsync(h->kscale, 0, sb, h->stream), -1);
     HIPCHK(hipMemsetAsync(h->vscale, 0, sb, h->stream), -1);
   }
-  h->kv_high = 0;
+  h->written.high = 0;
   megakernel_reset(h);
   return 0;
 }
