@@ -99,16 +99,14 @@ static int launch_step(BHandle* h, const BParams& p) {
       hipLaunchKernelGGL((bk_step<S, false>), dim3(h->G * STEP_WG_PER_CU), dim3(GT), 0, h->stream, g);
   }
   for (int l = 0; l < (h->step_variant == MK_BATCH_STEP_PERSISTENT ? 0 : L); ++l) {
-    hipLaunchKernelGGL((bk_qkv<S, PGroup1>), dim3(S::QKV / 16 * KS_QKV), dim3(GT), 0, h->stream, g, l);
+    hipLaunchKernelGGL((bk_qkv<S>), dim3(S::QKV / 16 * KS_QKV), dim3(GT), 0, h->stream, g, l);
     if (p.kscale)
-      hipLaunchKernelGGL((bk_attn<S, true, PGroup1>), dim3(BMAX * S::NKV * h->nsplit_max), dim3(AT), 0, h->stream, g,
-                         l);
+      hipLaunchKernelGGL((bk_attn<S, true>), dim3(BMAX * S::NKV * h->nsplit_max), dim3(AT), 0, h->stream, g, l);
     else
-      hipLaunchKernelGGL((bk_attn<S, false, PGroup1>), dim3(BMAX * S::NKV * h->nsplit_max), dim3(AT), 0, h->stream,
-                         g, l);
-    hipLaunchKernelGGL((bk_o<S, PGroup1>), dim3(S::H / 16 * KS_O), dim3(GT), 0, h->stream, g, l);
-    hipLaunchKernelGGL((bk_gu<S, PGroup1>), dim3(S::F / 16 * KS_GU), dim3(GT), 0, h->stream, g, l);
-    hipLaunchKernelGGL((bk_down<S, PGroup1>), dim3(S::H / 16 * KS_DN), dim3(GT), 0, h->stream, g, l);
+      hipLaunchKernelGGL((bk_attn<S, false>), dim3(BMAX * S::NKV * h->nsplit_max), dim3(AT), 0, h->stream, g, l);
+    hipLaunchKernelGGL((bk_o<S>), dim3(S::H / 16 * KS_O), dim3(GT), 0, h->stream, g, l);
+    hipLaunchKernelGGL((bk_gu<S>), dim3(S::F / 16 * KS_GU), dim3(GT), 0, h->stream, g, l);
+    hipLaunchKernelGGL((bk_down<S>), dim3(S::H / 16 * KS_DN), dim3(GT), 0, h->stream, g, l);
   }
   if (p.lmhead8)
     hipLaunchKernelGGL((bk_lm<S, true>), dim3(h->G), dim3(GT), 0, h->stream, p, lm_slot);
@@ -338,7 +336,6 @@ static int init_state(BHandle* h, const char* base, const long long* off, int n_
   p.inv_freq = inv;
   p.B = h->B, p.L = L, p.V = h->V;
   if (L >= 64) h->persistent_ok = false;  // the persistent step's split-K tags hold the layer in 6 bits
-  p.prefill = 0;
   HIPCHK(hipStreamSynchronize(h->stream), -1);
   return 0;
 }
@@ -451,26 +448,21 @@ static int run_steps(BHandle* h, const int* first, int n, int* out) {
 
 // The activation buffers of prefill column groups (group 0's at the slab's
 // start, group gi's gi * pf_gstride bytes later): offsets inside one group's
-// block, in BParams order x, xg, ssq, qkv, att, act, part, cnt, gpart, gcnt,
-// keys, rope.
-static long long group_layout(const BHandle* h, long long off[12]) {
-  // the prefill kernels keep no split-K sums (their GEMMs run the whole K) and
-  // one partial buffer for all groups (pf_part): part, gpart and gcnt get one
-  // line each, cnt (finished prefix splits per kv head) too
-  const long long sz[12] = {(long long)2 * BMAX * h->H * 4,
-                            (long long)4 * BMAX * h->H * 2,
-                            (long long)2 * (h->H / 16) * BMAX * 4,
-                            (long long)BMAX * h->QKV * 4,
-                            (long long)2 * BMAX * h->QD * 2,
-                            (long long)2 * BMAX * h->F * 2,
-                            256,
-                            256,
-                            256,
-                            256,
-                            (long long)BMAX * 8,
-                            (long long)BMAX * h->D * 4};
+// block, in BParams order x, xg, ssq, qkv, att, act, cnt (finished prefix
+// splits per kv head), keys, rope.
+constexpr int PG_BUFS = 9;
+static long long group_layout(const BHandle* h, long long off[PG_BUFS]) {
+  const long long sz[PG_BUFS] = {(long long)2 * BMAX * h->H * 4,
+                                 (long long)4 * BMAX * h->H * 2,
+                                 (long long)2 * (h->H / 16) * BMAX * 4,
+                                 (long long)BMAX * h->QKV * 4,
+                                 (long long)2 * BMAX * h->QD * 2,
+                                 (long long)2 * BMAX * h->F * 2,
+                                 256,
+                                 (long long)BMAX * 8,
+                                 (long long)BMAX * h->D * 4};
   long long o = 0;
-  for (int i = 0; i < 12; ++i) {
+  for (int i = 0; i < PG_BUFS; ++i) {
     off[i] = o;
     o += (sz[i] + 255) / 256 * 256;
   }
@@ -481,7 +473,7 @@ static long long group_layout(const BHandle* h, long long off[12]) {
 // larger one.
 static int ensure_groups(BHandle* h, int ng) {
   if (h->pf_groups >= ng) return 0;
-  long long off[12];
+  long long off[PG_BUFS];
   const long long stride = group_layout(h, off);
   if (h->pf_slab) {
     HIPCHK(hipStreamSynchronize(h->stream), -1);
@@ -527,7 +519,7 @@ static int prefill_passes(BHandle* h, int seq, const int* tokens, int n, int pos
   HIPCHK(hipEventRecord(h->ev0, h->stream), -1);
   const int ngt = (n + BMAX - 1) / BMAX, passes = (ngt + PG_MAX - 1) / PG_MAX;
   if (ensure_groups(h, ngt < PG_MAX ? ngt : PG_MAX)) return -1;
-  long long off[12];
+  long long off[PG_BUFS];
   group_layout(h, off);
   char* slab = h->pf_slab;
   for (int ps = 0; ps < passes; ++ps) {
@@ -538,9 +530,9 @@ static int prefill_passes(BHandle* h, int seq, const int* tokens, int n, int pos
     pp.x = reinterpret_cast<float*>(slab + off[0]), pp.xg = reinterpret_cast<uint16_t*>(slab + off[1]);
     pp.ssq = reinterpret_cast<float*>(slab + off[2]), pp.qkv = reinterpret_cast<float*>(slab + off[3]);
     pp.att = reinterpret_cast<uint16_t*>(slab + off[4]), pp.act = reinterpret_cast<uint16_t*>(slab + off[5]);
-    pp.part = h->pf_part, pp.cnt = reinterpret_cast<int*>(slab + off[7]);
-    pp.gpart = reinterpret_cast<float*>(slab + off[8]), pp.gcnt = reinterpret_cast<int*>(slab + off[9]);
-    pp.keys = reinterpret_cast<u64*>(slab + off[10]), pp.rope = reinterpret_cast<float*>(slab + off[11]);
+    pp.part = h->pf_part, pp.cnt = reinterpret_cast<int*>(slab + off[6]);
+    pp.gpart = nullptr, pp.gcnt = nullptr;
+    pp.keys = reinterpret_cast<u64*>(slab + off[7]), pp.rope = reinterpret_cast<float*>(slab + off[8]);
     // every column writes and reads this sequence's cache (FP8: byte index =
     // element index, so the sequence starts at byte seq * kv_seq)
     if (h->p.kscale) {
@@ -554,7 +546,6 @@ static int prefill_passes(BHandle* h, int seq, const int* tokens, int n, int pos
     }
     pp.kv_seq = 0;
     pp.sc_seq = 0;
-    pp.prefill = 1;
     pp.tok = h->pf_tok + c0;
     pp.pos = h->pf_pos + c0;
     pp.out = h->pf_out;

@@ -92,11 +92,12 @@ struct BParams {
   uint16_t* xg;             // [slot][2 consumers][2 planes][H/32][64][8] x * gain as bf16 hi / lo parts (unit_at):
                             //   consumer 0 = attn_norm of the next QKV (or final_norm), 1 = ffn_norm
   float* ssq;               // [slot][2 consumers][H/16][BMAX] sums of squares of x per 16-row block
-  float* qkv;               // [slot][BMAX][QKV] raw projections
+  float* qkv;               // [slot][BMAX][QKV] raw projections (a prefill: q normalised and rotated, k / v
+                            //   only in the cache; qkv_head)
   uint16_t* att;            // [slot][2][QD/32][64][8] merged attention output, bf16 hi / lo parts
   uint16_t* act;            // [slot][2][F/32][64][8] SiLU(g) * u, bf16 hi / lo parts
-  float* part;              // [BMAX][NKV][nsplit_max][PW] attention partials
-  int* cnt;                 // [BMAX][NKV] finished splits of the current layer
+  float* part;              // [BMAX][NKV][nsplit_max][PW] attention partials (a prefill: PC_WG of PC_PW floats)
+  int* cnt;                 // [BMAX][NKV] finished splits of the current layer (a prefill: [NKV] per group)
   float* gpart;             // split-K partial block sums of the GEMM kernels
   int* gcnt;                // [256] finished K splits per 16-row block
   u64* keys;                // [BMAX] argmax keys of the step
@@ -113,8 +114,6 @@ struct BParams {
   int* err;                 // bk_step: MK_ERR_TIMEOUT when a hand-off wait gave up
   unsigned long long timeout_ticks;  // bk_step: wall-clock ticks a hand-off wait may take
   int B, L, V, nsplit_max, max_steps;
-  int prefill;              // 1: the columns are consecutive prompt tokens of one sequence whose
-                            //    K / V the QKV kernel has already stored (kv_seq = 0, shared cache)
 };
 
 // Up to PG_MAX column groups that share one pass over the weights: a prefill
@@ -134,8 +133,9 @@ struct PGroupN {  // groups in the kernel argument
 };
 using PGroup1 = PGroupN<1>;  // the decode step
 // A prefill pass: group 0's parameters; group gi's activation buffers (x, xg,
-// ssq, qkv, att, act, part, cnt, gpart, gcnt, keys, rope) sit gi * gstride
-// bytes after group 0's, its tokens and positions 16 gi entries after them.
+// ssq, qkv, att, act, cnt, keys, rope) sit gi * gstride bytes after group 0's,
+// its tokens and positions 16 gi entries after them.  part is one buffer for
+// all groups; the GEMMs run the whole K and need no gpart / gcnt.
 struct PGroup {
   static constexpr int NG = PG_MAX;
   BParams p;
@@ -154,9 +154,8 @@ __host__ __device__ __forceinline__ BParams group_params(const PGroup& g, int gi
   const long long o = gi * g.gstride;
   BParams q = g.p;
   q.x = advance(q.x, o), q.xg = advance(q.xg, o), q.ssq = advance(q.ssq, o), q.qkv = advance(q.qkv, o);
-  q.att = advance(q.att, o), q.act = advance(q.act, o), q.part = advance(q.part, o), q.cnt = advance(q.cnt, o);
-  q.gpart = advance(q.gpart, o), q.gcnt = advance(q.gcnt, o), q.keys = advance(q.keys, o);
-  q.rope = advance(q.rope, o);
+  q.att = advance(q.att, o), q.act = advance(q.act, o), q.cnt = advance(q.cnt, o);
+  q.keys = advance(q.keys, o), q.rope = advance(q.rope, o);
   q.tok += BMAX * gi, q.pos += BMAX * gi;
   q.B = g.ntok - BMAX * gi < BMAX ? g.ntok - BMAX * gi : BMAX;
   return q;
@@ -676,31 +675,31 @@ __device__ __forceinline__ bool down_block(const BParams& p, int layer, int ep, 
   return true;
 }
 
-template <class S, class G>
-__global__ __launch_bounds__(GT) void bk_qkv(G p, int layer) {
+template <class S>
+__global__ __launch_bounds__(GT) void bk_qkv(PGroup1 p, int layer) {
   __shared__ float red[GW * 16 * 17];
   __shared__ float rr[RR_N];
   __shared__ int last;
   qkv_block<S, false>(group_of(p), layer, 0, blockIdx.x / KS_QKV, blockIdx.x % KS_QKV, red, rr, &last, NoWait{});
 }
 
-template <class S, class G>
-__global__ __launch_bounds__(GT) void bk_o(G p, int layer) {
+template <class S>
+__global__ __launch_bounds__(GT) void bk_o(PGroup1 p, int layer) {
   __shared__ float red[GW * 16 * 17];
   __shared__ int last;
   o_block<S, false>(group_of(p), layer, 0, blockIdx.x / KS_O, blockIdx.x % KS_O, red, &last, NoWait{});
 }
 
-template <class S, class G>
-__global__ __launch_bounds__(GT) void bk_gu(G p, int layer) {
+template <class S>
+__global__ __launch_bounds__(GT) void bk_gu(PGroup1 p, int layer) {
   __shared__ float red[GW * 16 * 17];
   __shared__ float rr[RR_N];
   __shared__ int last;
   gu_block<S, false>(group_of(p), layer, 0, blockIdx.x / KS_GU, blockIdx.x % KS_GU, red, rr, &last, NoWait{});
 }
 
-template <class S, class G>
-__global__ __launch_bounds__(GT) void bk_down(G p, int layer) {
+template <class S>
+__global__ __launch_bounds__(GT) void bk_down(PGroup1 p, int layer) {
   __shared__ float red[GW * 16 * 17];
   __shared__ int last;
   down_block<S, false>(group_of(p), layer, 0, blockIdx.x / KS_DN, blockIdx.x % KS_DN, red, &last, NoWait{});
@@ -1253,7 +1252,7 @@ __device__ __forceinline__ bool attn_item(const BParams& p, int layer, int ep, A
                      (w < 2 ? (g * 2 + w) * D : (w == 2 ? S::QD + g * D : S::QD + S::KVD + g * D));
   const float v0 = on ? src[l] : 0.f;
   float v = v0;
-  const bool own = on && !p.prefill && pos >= s * CH && pos < (s + 1) * CH;
+  const bool own = on && pos >= s * CH && pos < (s + 1) * CH;
   if (on && w < 3) {
     const float ss = wave_sum(v * v);
     const uint16_t* gn = p.norms + (long long)layer * S::NORM_STRIDE + (w < 2 ? S::NORM_Q : S::NORM_K);
@@ -1308,9 +1307,8 @@ __device__ __forceinline__ bool attn_item(const BParams& p, int layer, int ep, A
   for (int q = 0; q < NBW; ++q) {
     const int t0 = 32 * (s * AW * NBW + w + AW * q);
     if (t0 >= n) break;  // uniform over the wave (every block of an item that is off)
-    // position pos takes K / V from LDS (this item appended them; in a
-    // prefill the QKV kernel stored them before this kernel)
-    if (!p.prefill && pos >= t0 && pos < t0 + 32) {
+    // position pos takes K / V from LDS (this item appended them)
+    if (pos >= t0 && pos < t0 + 32) {
       const int rp = pos - t0;
       if constexpr (K8) {
         if (c16 == (rp & 15)) {  // register arrays take compile-time indices only
@@ -1501,9 +1499,9 @@ __device__ __forceinline__ bool attn_item(const BParams& p, int layer, int ep, A
 // step at KV 512-4096 has ~1,100 items; with four per CU the last ~10 % ran
 // as a second, latency-bound residency wave.
 constexpr int ATTN_WAVES_PER_EU = AT == 256 ? 5 : 2;
-template <class S, bool K8, class G>
+template <class S, bool K8>
 __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(ATTN_WAVES_PER_EU, ATTN_WAVES_PER_EU))) void bk_attn(
-    G pg, int layer) {
+    PGroup1 pg, int layer) {
   __shared__ AttnLds<S> sm;
   const BParams& p = group_of(pg);  // column group
   // workgroup i runs on XCD i % 8: every split of one (sequence, kv head)
@@ -1558,8 +1556,9 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(ATTN_WAVES_P
 constexpr int PC_NQ = 2 * BMAX;  // queries of a workgroup (a column group x 2 q heads)
 // Prefix splits (grid z): with few column groups a workgroup per (kv head,
 // group) leaves most of the chip idle, so the prefix is cut into up to PC_NZ
-// splits while there are at most PC_WG workgroups, each with at least two
-// blocks per wave; the split that finishes last merges (as in bk_attn).
+// splits while there are at most PC_WG workgroups and the last group, whose
+// prefix is the longest, keeps at least two blocks per wave (an earlier group's
+// splits may be shorter); the split that finishes last merges (as in bk_attn).
 constexpr int PC_WG = 256, PC_NZ = 16;
 constexpr int PC_PW = PC_NQ * 64 + 2 * PC_NQ;  // floats of a split's partial: o[32][64], max[32], sum[32]
 template <class S, bool K8>
