@@ -134,14 +134,15 @@ float megakernel_last_kernel_ms(void* handle);
 int megakernel_grid_size(void* handle);
 
 /* Minimum positions per attention work item (default 512; 256 for head_dim
- * 128). */
+ * 128).  A launch of the automatic kernel choice may take larger items to
+ * stay in the class kernel (MK_KERNEL_AUTO below). */
 int megakernel_set_attention_chunk(void* handle, int chunk_min);
 
-/* Above this many attention splits per kv head (default 20: contexts beyond
- * 10,240 positions at the default chunk) the workgroup of each head's first
- * split merges the head's splits and the O phase reads one merged partial; at
- * or below it every O workgroup merges the splits itself.  Tuning and testing
- * only. */
+/* Above this many attention splits per kv head (default 20: at the default
+ * chunk, contexts beyond 10,240 positions, 5,120 for head_dim 128) the
+ * workgroup of each head's first split merges the head's splits and the O
+ * phase reads one merged partial; at or below it every O workgroup merges the
+ * splits itself.  Tuning and testing only. */
 int megakernel_set_attention_merge(void* handle, int merge_min);
 
 /* Which persistent kernel decodes (no counterpart in the reference, whose

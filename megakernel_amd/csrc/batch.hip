@@ -129,18 +129,19 @@ static void launch_pgemm(BHandle* h, const PGroup& g, int l) {
 
 // Tile shapes by the pass's column groups n: the largest that still gives the
 // chip about one workgroup per CU -- a larger tile reads fewer bytes per
-// product, a smaller one starts more workgroups.  (us per layer at n = 2 / 4 /
-// 8 / 16 / 32 / 64; * the range it is used in.)
-//   QKV   2x1   4.4*  4.7*  5.5   7.9  13.6  24.9     O    2x1  4.1*  3.8*  3.9*  5.1   8.2  15.9
-//         2x2   4.6   5.1   5.1*  6.6  10.6  19.0          2x2  4.5   4.4   4.3   4.6*  6.7  11.7
-//         4x2   5.2   5.1   5.2   5.5*  9.5  18.1          4x2  5.0   4.9   5.0   5.1   5.8* 11.1
-//         4x4   6.1   6.7   6.8   7.0   7.8* 13.1          4x4  6.3   6.7   6.8   6.9   7.3   9.6*
-//         8x4   9.2  10.1  10.2  10.5  10.8  12.1*
-//   gate  2x1   6.2*  7.6   9.6  15.3  25.0  46.0     down 1x1  5.1*  5.2*  8.2  14.9  28.1  53.1
-//   / up  2x2   7.3   7.0*  8.9* 11.7* 18.6  30.5          2x1  6.1   6.1   6.3* 11.2  21.3  40.4
-//         2x4   8.0   9.5   9.1  12.0  16.5* 27.6*         2x2  7.5   7.5   7.4   8.0* 15.2  28.1
-//         4x4  11.2  13.2  12.9  12.6  21.6  31.8          4x2  9.6   9.5   9.3   9.7  11.5* 19.7
-//                                                          4x4 10.9  13.5  13.0  13.4  15.1  18.4*
+// product, a smaller one starts more workgroups.  (Median us per launch inside
+// whole passes under the kernel trace, epilogues included, at n = 2 / 4 / 8 /
+// 16 / 32 / 64; * the range it is used in, - not told apart from n = 2.  8x4 and
+// 4x4 of QKV are equal at 64.)
+//   QKV   4x1   6.9*  6.7*  6.7* 10.2  17.2  31.1     O    2x1  5.0*  5.0*  5.0*  5.8   9.1  16.0
+//         4x2   8.2   7.9   7.7   7.6* 13.1  23.8          2x2  5.8   5.6   5.4   5.4*  7.6  11.8
+//         4x4   9.1    -    8.9   8.6   9.0* 14.0          4x2  6.8   6.6   6.5   6.4   7.0* 11.7
+//         8x4  13.4    -   13.4  12.7  12.9  14.1*         4x4  8.5    -    8.4   8.0   8.5  10.2*
+//   gate  2x1   6.7*  8.3  10.3  15.9  26.0  46.4     down 1x1  6.8*  6.6*  9.8  15.9  28.4  53.4
+//   / up  2x2   7.6   7.5*  9.6* 12.2* 19.4  32.2          2x1  8.5   8.2   8.2* 13.1  22.8  42.0
+//         2x4   9.8    -   10.1  12.3  17.4* 29.3*         2x2 11.1  10.5  10.1  10.0* 16.6  29.6
+//         4x4  13.5    -   13.6  12.7  22.0  32.3          4x2 14.7  14.0  13.2  12.8  13.1* 22.6
+//                                                          4x4 19.2    -   18.4  17.5  18.2  19.8*
 template <class S>
 static void launch_pgemm_qkv(BHandle* h, const PGroup& g, int l) {
   if (g.n <= 8) launch_pgemm<S, PT_QKV, PTile<4, 1, 4, 1, 8>>(h, g, l);

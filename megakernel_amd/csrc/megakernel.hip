@@ -425,7 +425,12 @@ struct Handle {
   int max_launch_tokens = 0;
   int nsplit_max = 1, chunk_min = 256 * KVB;  // the blocks a workgroup's waves hold in registers
   int chunk_eff = 0;                           // the attention chunk of the last launch (launch_chunk)
-  int merge_min = 20;  // above this many splits per kv head the first split's workgroup merges them
+  // above this many splits per kv head the first split's workgroup merges them
+  // (set with splits of 512 positions.  head_dim 128, 256 positions, us per
+  // token, every O workgroup / the first split: 12 splits 510 / 560, 16 547 /
+  // 561, 20 592 / 565, 21 619 / 562, 26 866 / 573; FP8 cache 503 / 530, 541 /
+  // 526, 583 / 528, 610 / 528, 811 / 536)
+  int merge_min = 20;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   float last_ms = 0.f;
@@ -633,8 +638,13 @@ static Handle* create(int preset, int vocab, int max_seq) {
       break;
     case PRESET_QWEN3_06B:
       h->sh = shape_info<ShapeQwen3>();
-      // (measured at 300 / 700 / 2,500 / 6,000 positions, us per token: splits
-      // of 256 446 / 460 / 503 / 571, of 512 494 / 505 / 563 / 620)
+      // (us per token with splits of 256 against 512 positions: spread kernel
+      // at 300 / 700 / 2,500 / 6,000 positions 446 / 460 / 503 / 571 against
+      // 494 / 505 / 563 / 620; automatic choice at 700 / 1,500 / 4,060 / 8,100 /
+      // 12,000 357 / 438 / 547 / 621 / 682 against 408 / 462 / 571 / 658 / 707,
+      // FP8 cache 369 / 439 / 541 / 579 / 630 against 411 / 457 / 554 / 626 /
+      // 628; it loses up to 2 %, at 1,700, 466 against 457.  From 16,384
+      // positions on both are 32 splits and equal)
       h->chunk_min = 256 * kv_blocks<ShapeQwen3>();
       h->launch = launch_decode_qwen3;
       h->has_cls = true;
@@ -1353,7 +1363,7 @@ int megakernel_set_layer_fp8(void* handle, int enable) {
     return -1;
   }
   if (enable && (!h->has_w8 || !h->roles_ok[1])) {
-    mk::set_err("FP8 layer weights need the class kernel, which this preset / device does not have");
+    mk::set_err("FP8 layer weights need the FP8 form of the class kernel, which this preset / device does not have");
     return -1;
   }
   if (enable && !h->layers8) {

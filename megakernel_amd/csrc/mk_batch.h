@@ -719,17 +719,19 @@ __global__ __launch_bounds__(GT) void bk_down(PGroup1 p, int layer) {
 // the epilogue's inputs are loaded before the product.
 //
 // What bounds it: a short pass the latency of one load round per kernel (23
-// tokens: 4 - 6 us per GEMM, a kernel's fixed cost about 4), a long one the
+// tokens: 5 - 7 us per GEMM, a kernel's fixed cost about 4), a long one the
 // bytes that cross L2 per product.  No barrier and no LDS copy stands between
 // a load and its product, and a wave's loads are all independent, so a
 // workgroup keeps 64 - 256 KiB in flight.  The kernels before this staged both
 // operands in LDS by chunks of K, with a barrier per chunk: every chunk waited
-// for its loads (0.5 - 1.2 us each, 16 to 32 in a row).  us per layer, before
-// -> now:            2 groups     13           32           64
-//   QKV              9.3 -> 4.4   9.6 -> 5.4   10.1 -> 7.8  15.0 -> 12.1
-//   O                8.0 -> 3.8   8.2 -> 4.5    8.7 -> 5.8  11.0 -> 9.6
-//   gate / up       18.7 -> 6.2  23.5 -> 11.4  25.9 -> 16.5 32.5 -> 27.6
-//   down            19.2 -> 5.1  18.3 -> 7.4   19.9 -> 11.5 20.7 -> 18.4
+// for its loads (0.5 - 1.2 us each, 16 to 32 in a row).  us per layer inside
+// whole passes (kernel trace), the LDS-tiled kernels on row-major planes -> now
+// (QKV: before, its append kernel added; now, with the head epilogue):
+//                    2 groups      13            32            64
+//   QKV             14.4 -> 7.0   15.0 -> 8.1   15.6 -> 9.4   21.6 -> 14.7
+//   O               11.6 -> 5.0   12.2 -> 5.2   12.7 -> 7.3   18.6 -> 10.5
+//   gate / up       20.7 -> 7.0   26.6 -> 12.8  31.1 -> 18.0  38.2 -> 30.8
+//   down            25.6 -> 7.1   24.8 -> 9.7   25.9 -> 13.3  31.5 -> 20.3
 template <int MR_, int NG_, int CW_, int NBUF_, int W_>
 struct PTile {
   static constexpr int MR = MR_, NG = NG_, CW = CW_, NBUF = NBUF_, W = W_;
@@ -1544,10 +1546,10 @@ __global__ __launch_bounds__(AT) __attribute__((amdgpu_waves_per_eu(ATTN_WAVES_P
 // What bounds it: the vector work beside the products (about 1,000 cycles of
 // softmax and splitting per block step against 768 of matrix products) and,
 // for a few groups, the load round trip of a wave's next block; two waves per
-// SIMD.  us per layer, 64 groups at position 0 / 1,024 / 3,072: 19.1 / 34.5 /
-// 63.7 with 8-byte V loads, non-temporal loads and one query tile after the
-// other, 15.2 / 27.0 / 50.5 as it is; FP8 23.7 / 43.5 / 82.7 and 16.3 / 30.4 /
-// 57.1; 13 groups at 1,500: 17.0 and 14.7.
+// SIMD.  us per layer inside whole passes (kernel trace), 64 groups at position
+// 0 / 1,024 / 3,072: 20.4 / 36.5 / 66.5 with 8-byte V loads, non-temporal loads
+// and one query tile after the other, 17.2 / 30.2 / 55.8 as it is; FP8 23.8 /
+// 43.1 / 82.2 and 17.6 / 32.1 / 60.8; 13 groups at 1,500: 16.9 and 15.4.
 // (Earlier measurements: three K / V register sets 23.2 against two 20.6; two
 // parts 20.8 against three 21.6.)
 #ifndef MK_PATTN_NPART
