@@ -359,7 +359,8 @@ def test_fp8_layers_lmhead_and_kv_together():
 def test_fp8_layers_need_class_kernel():
     """FP8 layer weights are served by the class-specialised kernel only: the
     spread kernel variant refuses the launch with a message, the QWEN3 preset
-    (no class kernel) refuses the switch, and the handle keeps working."""
+    (whose class kernel has no FP8-weight form) refuses the switch, and the
+    handle keeps working."""
     from megakernel_amd import _lib
     eng, orc, dw = make_pair(BASELINE_2L, 67, 64)
     try:

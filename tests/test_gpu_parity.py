@@ -647,7 +647,9 @@ def test_qwen3_context_ranges(ctx, kv8):
 def test_reset_clears_every_written_row(kv8):
     """reset zeroes the cache up to the highest row written since the last
     clear, whichever path wrote it, at block edges and at the capacity; a
-    change of format clears what the other format held."""
+    change of format clears what the other format held.  With an FP8 cache what
+    is read back is code x scale: that the codes are zero shows, that the
+    scales are does not (no call reads them alone)."""
     shape = TINY
     dw = DeviceWeights(shape, 3)
     eng = MegakernelEngine(shape=shape, max_seq=96, device_weights=dw, prefill=True)
